@@ -194,7 +194,8 @@ __global__ __launch_bounds__(64) void k_mlp_train(MlpDev m, const float *__restr
             const uint16_t b = bf16_bits(v);
             x[r * kStrideIn + c] = b;
             xT[c * kStrideT + r] = b;
-            tg[r][c] = ok ? targets[(size_t)sid * kMlpRad + c] : 0.0f;
+            // a target row has kMlpRad (48) values, fewer than the feature row
+            if (c < kMlpRad) tg[r][c] = ok ? targets[(size_t)sid * kMlpRad + c] : 0.0f;
         }
         for (int i = lane; i < (64 - kMlpIn) * 32; i += 64) xT[(kMlpIn + i / 32) * kStrideT + (i % 32)] = 0;  // pad rows kMlpIn..63
         __syncthreads();

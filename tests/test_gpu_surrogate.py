@@ -446,3 +446,27 @@ def test_train_cli_on_dump_files(rc, tmp_path):
         st.run_device(depth, emis, irr)
         torch.cuda.synchronize()
         assert torch.isfinite(irr).all()
+
+
+def test_gradient_reads_only_its_targets(rc):
+    """Targets that end where their allocation ends (65,536 rows = 12 MiB, a
+    block of their own) give the same gradient as the head of a longer buffer:
+    the kernel reads 48 values of a row, not the feature row's 64."""
+    params, mean, istd, scale = _net(7)
+    n = 65536
+    x, t = _rand_io(n, 4)
+    xd = torch.from_numpy(x).cuda()
+    exact_fit = torch.empty((n, rc._abi.MLP_RADIANCE), dtype=torch.float32, device="cuda:0")
+    exact_fit.copy_(torch.from_numpy(t))
+    longer = torch.full((n + 64, rc._abi.MLP_RADIANCE), float("nan"), device="cuda:0")
+    longer[:n] = exact_fit
+    got = []
+    with rc.RadianceCascadeStage(64, 64, levels=3) as st:
+        st.mlp_set(params, mean, istd, scale)
+        for td in (exact_fit, longer[:n]):
+            grad = torch.empty(rc._abi.MLP_PARAMS, dtype=torch.float32, device="cuda:0")
+            lo = torch.empty(1, dtype=torch.float32, device="cuda:0")
+            st.mlp_gradient(xd, td, grad, lo)
+            got.append((grad.cpu(), lo.cpu()))
+    assert torch.isfinite(got[1][0]).all()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
