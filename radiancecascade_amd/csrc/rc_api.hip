@@ -81,7 +81,6 @@ struct rc_ctx {
     uint32_t train_scenes = 0;
     int adam_t = 0;
     float *mlp_partial = nullptr, *mlp_loss_part = nullptr;
-    int *mlp_idx = nullptr;
     int mlp_cap_rows = 0;
     bool surr_alloc = false;
     MipArgs mip{};
@@ -520,12 +519,11 @@ static rc_status run_frame(rc_ctx *c, const float *depth, const float *emissive,
 static void free_mlp(rc_ctx *c)
 {
     void *p[] = {c->mlp.master, c->mlp.adam_m, c->mlp.adam_v, c->mlp.wt, c->mlp.wk, c->mlp.bias, c->mlp.in_mean,
-                 c->mlp.in_istd, c->mlp_partial, c->mlp_loss_part, c->mlp_idx};
+                 c->mlp.in_istd, c->mlp_partial, c->mlp_loss_part};
     for (void *q : p)
         if (q) hipFree(q);
     c->mlp = MlpDev{};
     c->mlp_partial = c->mlp_loss_part = nullptr;
-    c->mlp_idx = nullptr;
     c->mlp_cap_rows = 0;
     if (c->flag_host) hipHostFree(c->flag_host);
     c->flag_host = nullptr;
@@ -1617,29 +1615,21 @@ rc_status rc_mlp_gradient(rc_ctx *c, const float *feats, const float *targets, u
     const int parts = (int)((n + 31) / 32);
     rc_status st = ensure_mlp_scratch(c, parts, (int)n);
     if (st != RC_OK) return st;
-    if ((int)n > 0) {
-        if (c->mlp_idx) hipFree(c->mlp_idx);
-        c->mlp_idx = nullptr;
-        std::vector<int> idx(n);
-        for (uint32_t i = 0; i < n; ++i) idx[i] = (int)i;
-        HIP_TRY(c, hipMalloc(&c->mlp_idx, n * sizeof(int)));
-        HIP_TRY(c, hipMemcpy(c->mlp_idx, idx.data(), n * sizeof(int), hipMemcpyHostToDevice));
-    }
-    HIP_TRY(c, launch_mlp_train(c->mlp, feats, targets, c->mlp_idx, (int)n, 1, c->mlp_partial, c->mlp_loss_part, parts,
-                                s));
-    HIP_TRY(c, launch_mlp_reduce(c->mlp_partial, parts, grad, s));
-    HIP_TRY(c, launch_sum_f32(c->mlp_loss_part, parts, loss, s));
-    HIP_TRY(c, hipStreamSynchronize(s));
+    HIP_TRY(c, launch_mlp_train(c->mlp, feats, targets, nullptr, (int)n, 1, c->mlp_partial, c->mlp_loss_part, parts, s));
+    HIP_TRY(c, launch_mlp_reduce(c->mlp_partial, c->mlp_loss_part, parts, grad, loss, s));
     return RC_OK;
 }
 
-static rc_status adam_step(rc_ctx *c, const float *grad, float lr, hipStream_t s)
+// The next Adam step's decay rates and bias corrections.
+static void adam_next(rc_ctx *c, float &b1, float &b2, float &eps, float &c1, float &c2)
 {
-    const double b1 = 0.9, b2 = 0.999;
+    const double d1 = 0.9, d2 = 0.999;
     c->adam_t += 1;
-    const float c1 = (float)(1.0 - pow(b1, c->adam_t)), c2 = (float)(1.0 - pow(b2, c->adam_t));
-    HIP_TRY(c, launch_mlp_adam(c->mlp, grad, lr, (float)b1, (float)b2, 1e-8f, c1, c2, s));
-    return RC_OK;
+    b1 = (float)d1;
+    b2 = (float)d2;
+    eps = 1e-8f;
+    c1 = (float)(1.0 - pow(d1, c->adam_t));
+    c2 = (float)(1.0 - pow(d2, c->adam_t));
 }
 
 rc_status rc_mlp_adam(rc_ctx *c, const float *grad, float lr, void *stream)
@@ -1647,9 +1637,11 @@ rc_status rc_mlp_adam(rc_ctx *c, const float *grad, float lr, void *stream)
     if (!c || !grad) return fail(c, RC_ERR_NULL, "rc_mlp_adam: NULL argument");
     if (!c->mlp_ready) return fail(c, RC_ERR_STATE, "rc_mlp_adam: no network");
     HIP_TRY(c, hipSetDevice(c->cfg.device));
-    rc_status st = adam_step(c, grad, lr, (hipStream_t)stream);
-    if (st == RC_OK) drop_graph(c);
-    return st;
+    float b1, b2, eps, c1, c2;
+    adam_next(c, b1, b2, eps, c1, c2);
+    HIP_TRY(c, launch_mlp_adam(c->mlp, grad, lr, b1, b2, eps, c1, c2, (hipStream_t)stream));
+    drop_graph(c);
+    return RC_OK;
 }
 
 rc_status rc_surrogate_samples(rc_ctx *c, const rc_gbuffer *g, float *feats, float *targets, void *stream)
@@ -1770,7 +1762,7 @@ static rc_status train_rows(rc_ctx *c, const float *feats, float *targets, size_
     hipStream_t s = nullptr;
     double *stats = nullptr;
     int *idx = nullptr;
-    float *partial = nullptr, *loss_part = nullptr, *grad = nullptr, *step_loss = nullptr;
+    float *partial = nullptr, *loss_part = nullptr, *step_loss = nullptr;
     rc_status st;
     // normalisation: per-input mean and std, one RMS scale for the targets
     const int parts = 1024;
@@ -1817,8 +1809,6 @@ static rc_status train_rows(rc_ctx *c, const float *feats, float *targets, size_
     owned.push_back(partial);
     HIP_TRY(c, hipMalloc(&loss_part, (size_t)wgs * sizeof(float)));
     owned.push_back(loss_part);
-    HIP_TRY(c, hipMalloc(&grad, kMlpParams * sizeof(float)));
-    owned.push_back(grad);
     HIP_TRY(c, hipMalloc(&step_loss, steps * sizeof(float)));
     owned.push_back(step_loss);
     std::vector<int> perm(N);
@@ -1840,10 +1830,9 @@ static rc_status train_rows(rc_ctx *c, const float *feats, float *targets, size_
         const float lr = cfg->lr * powf(cfg->lr_decay > 0.0f ? cfg->lr_decay : 1.0f, (float)e);
         for (size_t k = 0; k < steps; ++k) {
             HIP_TRY(c, launch_mlp_train(c->mlp, feats, targets, idx + k * batch, batch, nb, partial, loss_part, wgs, s));
-            HIP_TRY(c, launch_mlp_reduce(partial, wgs, grad, s));
-            HIP_TRY(c, launch_sum_f32(loss_part, wgs, step_loss + k, s));
-            st = adam_step(c, grad, lr, s);
-            if (st != RC_OK) return st;
+            float b1, b2, eps, c1, c2;
+            adam_next(c, b1, b2, eps, c1, c2);
+            HIP_TRY(c, launch_mlp_reduce_adam(c->mlp, partial, loss_part, wgs, step_loss + k, lr, b1, b2, eps, c1, c2, s));
         }
         HIP_TRY(c, hipMemcpy(hl.data(), step_loss, steps * sizeof(float), hipMemcpyDeviceToHost));
         double tot = 0.0;

@@ -309,13 +309,18 @@ struct MlpDev {
 };
 
 hipError_t launch_mlp_infer(const MlpDev &m, const float *feats, int n, float *out, hipStream_t s);
+// idx: sample ids, or nullptr for rows 0 .. batch - 1
 hipError_t launch_mlp_train(const MlpDev &m, const float *feats, const float *targets, const int *idx, int batch,
                             int nb, float *partial, float *loss_part, int parts, hipStream_t s);
-hipError_t launch_mlp_reduce(const float *partial, int parts, float *grad, hipStream_t s);
+// gradient and loss from the workgroups' partial sums, in workgroup order
+hipError_t launch_mlp_reduce(const float *partial, const float *loss_part, int parts, float *grad, float *loss,
+                             hipStream_t s);
+// the same sums and the Adam step with them (the gradient is not stored)
+hipError_t launch_mlp_reduce_adam(const MlpDev &m, const float *partial, const float *loss_part, int parts, float *loss,
+                                  float lr, float b1, float b2, float eps, float c1, float c2, hipStream_t s);
 hipError_t launch_mlp_adam(const MlpDev &m, const float *grad, float lr, float b1, float b2, float eps, float c1,
                            float c2, hipStream_t s);
 hipError_t launch_mlp_refresh(const MlpDev &m, hipStream_t s);
-hipError_t launch_sum_f32(const float *x, int n, float *out, hipStream_t s);
 
 // ---- surrogate far field (rc_surrogate.hip) ---------------------------------
 // Emitter / occluder mip pyramid: level m (1..levels) has cells of 2^m x 2^m

@@ -24,6 +24,7 @@
 namespace rc {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 // ---- parameter layout ---------------------------------------------------------
@@ -156,195 +157,326 @@ __global__ __launch_bounds__(kBlock) void k_mlp_infer(MlpDev m, const float *__r
 }
 
 // ---- training: forward + backward, per-workgroup gradient partials -----------
-// One wave per workgroup; the workgroup takes `nb` 32-sample blocks of the
-// batch (sample ids from idx) and writes the FP32 sum of their gradients to
-// partial[blockIdx.x][kMlpParams] (bias gradients included) and its loss sum.
-// Targets are normalised [n][48].  Weights are read from global memory (L2).
-__global__ __launch_bounds__(64) void k_mlp_train(MlpDev m, const float *__restrict__ feats,
-                                                  const float *__restrict__ targets, const int *__restrict__ idx,
-                                                  int batch, int nb, float *__restrict__ partial,
-                                                  float *__restrict__ loss_part)
+// A workgroup of 4 waves takes `nb` 32-sample blocks of the batch (sample ids
+// from idx, or consecutive rows) and writes the FP32 sum of their gradients to
+// partial[blockIdx.x][kMlpParams] and its loss sum.  Targets are normalised
+// [n][48].  Waves 0 and 1 own the two 32-column tiles of every layer's
+// output (and of the upstream gradient dA), their weight fragments held in
+// registers; each of the 4 waves owns one 32x32 tile of every dW; wave 3 sums
+// the bias gradients.
+//
+// What bounds it: 88 MFMAs a block take under a microsecond, the rest is the
+// chain of about a dozen barrier-separated LDS steps, so the aim is many
+// blocks in flight (64 KB of LDS: 2 workgroups, 8 waves per CU) and no global
+// round trip inside a block; after that the 66.5 KB of partial sums each
+// workgroup writes (34 MB for 16,384 samples).  The block size stays 32 samples
+// (and the partials one per block) because the gradient is defined as the sum
+// of the blocks' FP32 sums in block order.  Partials are written in the
+// accumulators' own order (dw_part_index), 1 KB per store, and put in master
+// order by the reduction.  16,384 samples: 85 us with one
+// wave per block (weights read from L2 per product, scalar LDS copies), 20 us so.
+constexpr int kTrainRow = 64 + 1, kTrainTgt = kMlpRad + 1;
+
+// Where element i of a workgroup's partial belongs in the master vector: dW
+// of layer l as 4 tiles of 32x32 in accumulator order ([tile][v / 4][lane][v %
+// 4], tile 2 mt + nt: outputs 32 mt.., inputs 32 nt..), then the biases.
+__device__ inline int part_to_master(int i)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t x[32 * kStrideIn], h1[32 * kStrideHid], h2[32 * kStrideHid],
-        h3[32 * kStrideHid];
-    __shared__ __attribute__((aligned(16))) uint16_t xT[64 * kStrideT], hT1[64 * kStrideT], hT2[64 * kStrideT],
-        hT3[64 * kStrideT];
+    static_assert(kMlpIn == 64 && kMlpHid == 64, "square layers");
+    if (i >= 4 * 4096) {
+        const int b = i - 4 * 4096;
+        return mlp_p_b(0) + (b >> 6) * (64 * 64 + 64) + (b & 63);
+    }
+    const int l = i >> 12, t = (i >> 10) & 3, q = (i >> 8) & 3, lane = (i >> 2) & 63, j = i & 3;
+    const int o = (t >> 1) * 32 + 8 * q + 4 * (lane >> 5) + j, in = (t & 1) * 32 + (lane & 31);
+    return mlp_p_w(0) + l * (64 * 64 + 64) + in * 64 + o;
+}
+
+__global__ __launch_bounds__(kBlock, 2) void k_mlp_train(MlpDev m, const float *__restrict__ feats,
+                                                         const float *__restrict__ targets,
+                                                         const int *__restrict__ idx, int batch, int nb,
+                                                         float *__restrict__ partial, float *__restrict__ loss_part)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t act[4][32 * kStrideHid];  // inputs of layers 0..3 [sample][feature]
+    __shared__ __attribute__((aligned(16))) uint16_t actT[4][64 * kStrideT];   // the same [feature][sample]
     __shared__ __attribute__((aligned(16))) uint16_t g[32 * kStrideHid], gT[64 * kStrideT];
-    __shared__ float zs[32][kMlpOut + 1];
-    __shared__ float tg[32][kMlpRad + 1];
-    __shared__ float gsum[64];
-    const int lane = threadIdx.x;
-    const uint16_t *wt[4] = {m.wt, m.wt + 64 * kMlpIn, m.wt + 64 * kMlpIn + 64 * kMlpHid,
-                             m.wt + 64 * kMlpIn + 2 * 64 * kMlpHid};
-    const uint16_t *wk[4] = {m.wk, m.wk + 64 * kMlpIn, m.wk + 64 * kMlpIn + 64 * kMlpHid,
-                             m.wk + 64 * kMlpIn + 2 * 64 * kMlpHid};
-    float *part = partial + (size_t)blockIdx.x * kMlpParams;
+    __shared__ float zs[32 * kTrainRow];  // outputs, then the FP32 upstream gradient
+    __shared__ float tg[32 * kTrainTgt];
+    __shared__ float gerr[32];            // dL/dz_48
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int c32 = lane & 31, half = lane >> 5;
+    const int oc = (wave & 1) * 32 + c32;  // the column of this lane in its wave's output tile
+    bf16x8 wf[4][4], wb[3][4];
+    float bias[4] = {0.f, 0.f, 0.f, 0.f};
+    if (wave < 2) {
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            bias[l] = m.bias[l * 64 + oc];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                wf[l][i] = ld8(m.wt + mlp_w_off(l) + oc * 64 + 16 * i + 8 * half);
+                if (l > 0) wb[l - 1][i] = ld8(m.wk + mlp_w_off(l) + oc * 64 + 16 * i + 8 * half);
+            }
+        }
+    }
+    const float mean = m.in_mean[lane], istd = m.in_istd[lane];
+    float *const part = partial + (size_t)blockIdx.x * kMlpParams;
     float loss_acc = 0.0f;
     const float inv_bn = 1.0f / ((float)batch * kMlpRad), inv_b = 1.0f / (float)batch;
 
     for (int bi = 0; bi < nb; ++bi) {
-        const int s0 = (blockIdx.x * nb + bi) * 32;
-        // features (normalised) -> x and xT; targets -> tg.  Rows past the
-        // batch are zero features with zero gradient.
-        for (int i = lane; i < 32 * kMlpIn; i += 64) {
-            const int r = i / kMlpIn, c = i % kMlpIn;
-            const bool ok = s0 + r < batch;
-            const int sid = ok ? idx[s0 + r] : 0;
-            const float v = ok ? (feats[(size_t)sid * kMlpIn + c] - m.in_mean[c]) * m.in_istd[c] : 0.0f;
-            const uint16_t b = bf16_bits(v);
-            x[r * kStrideIn + c] = b;
-            xT[c * kStrideT + r] = b;
-            // a target row has kMlpRad (48) values, fewer than the feature row
-            if (c < kMlpRad) tg[r][c] = ok ? targets[(size_t)sid * kMlpRad + c] : 0.0f;
+        const int s0 = ((int)blockIdx.x * nb + bi) * 32;
+        // features (normalised) and targets of rows 8 wave .. 8 wave + 7, a
+        // column per lane, all loads in flight at once.  Rows past the batch
+        // are zero features with zero gradient.
+        {
+            float f[8], t[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int r = s0 + 8 * wave + j;
+                const bool ok = r < batch;
+                const size_t sid = ok ? (idx ? (size_t)idx[r] : (size_t)r) : 0;
+                f[j] = ok ? feats[sid * kMlpIn + lane] : 0.0f;
+                t[j] = ok && lane < kMlpRad ? targets[sid * kMlpRad + lane] : 0.0f;
+            }
+            uint32_t b[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                b[j] = s0 + 8 * wave + j < batch ? bf16_bits((f[j] - mean) * istd) : 0;
+                act[0][(8 * wave + j) * kStrideHid + lane] = (uint16_t)b[j];
+                if (lane < kMlpRad) tg[(8 * wave + j) * kTrainTgt + lane] = t[j];
+            }
+            *reinterpret_cast<uint4 *>(&actT[0][lane * kStrideT + 8 * wave]) =
+                make_uint4(b[0] | b[1] << 16, b[2] | b[3] << 16, b[4] | b[5] << 16, b[6] | b[7] << 16);
         }
-        for (int i = lane; i < (64 - kMlpIn) * 32; i += 64) xT[(kMlpIn + i / 32) * kStrideT + (i % 32)] = 0;  // pad rows kMlpIn..63
         __syncthreads();
-        floatx16 z[2];
-        mlp_forward32(x, h1, h2, h3, wt, m.bias, z, hT1, hT2, hT3);
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
+        for (int l = 0; l < 4; ++l) {
+            if (wave < 2) {
+                floatx16 c = {};
 #pragma unroll
-            for (int v = 0; v < 16; ++v) zs[acc_row(v, lane)][nt * 32 + (lane & 31)] = z[nt][v];
-        __syncthreads();
+                for (int i = 0; i < 4; ++i)
+                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(act[l] + c32 * kStrideHid + 16 * i + 8 * half),
+                                                                wf[l][i], c, 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int row = 8 * q + 4 * half;
+                    if (l == 3) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) zs[(row + j) * kTrainRow + oc] = c[4 * q + j] + bias[3];
+                    } else {
+                        uint32_t h[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            h[j] = bf16_bits(fmaxf(c[4 * q + j] + bias[l], 0.0f));
+                            act[l + 1][(row + j) * kStrideHid + oc] = (uint16_t)h[j];
+                        }
+                        *reinterpret_cast<uint2 *>(&actT[l + 1][oc * kStrideT + row]) =
+                            make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+                    }
+                }
+            }
+            __syncthreads();
+        }
 
-        // dL/dz4 per row: lanes 0..31 own one sample each (FP32, deterministic)
-        if (lane < 32) {
+        // loss and the error head's gradient: lanes 0..31 of wave 0 own one
+        // sample each (FP32, fixed order)
+        if (threadIdx.x < 32) {
             const bool ok = s0 + lane < batch;
+            const float *z = zs + lane * kTrainRow, *t = tg + lane * kTrainTgt;
             float se = 0.0f;
+#pragma unroll 16
             for (int c = 0; c < kMlpRad; ++c) {
-                const float d = zs[lane][c] - tg[lane][c];
+                const float d = z[c] - t[c];
                 se = fmaf(d, d, se);
             }
-            const float e_t = logf(se * (1.0f / kMlpRad) + kMlpErrEps);
-            const float de = zs[lane][kMlpErr] - e_t;
+            const float de = z[kMlpErr] - logf(se * (1.0f / kMlpRad) + kMlpErrEps);
             if (ok) loss_acc += se * inv_bn + kMlpErrWeight * de * de * inv_b;
-            for (int c = 0; c < kMlpOut; ++c) {
+            gerr[lane] = ok ? kMlpErrWeight * 2.0f * de * inv_b : 0.0f;
+        }
+        __syncthreads();
+        {
+            // dL/dz4 of rows 8 wave.., a column per lane
+            uint32_t b[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int r = 8 * wave + j;
                 float gv = 0.0f;
-                if (ok && c < kMlpRad) gv = 2.0f * (zs[lane][c] - tg[lane][c]) * inv_bn;
-                if (ok && c == kMlpErr) gv = kMlpErrWeight * 2.0f * de * inv_b;
-                zs[lane][c] = gv;  // reuse as the FP32 gradient
+                if (s0 + r < batch) {
+                    if (lane < kMlpRad) gv = 2.0f * (zs[r * kTrainRow + lane] - tg[r * kTrainTgt + lane]) * inv_bn;
+                    else if (lane == kMlpErr) gv = gerr[r];
+                }
+                zs[r * kTrainRow + lane] = gv;
+                b[j] = bf16_bits(gv);
+                g[r * kStrideHid + lane] = (uint16_t)b[j];
             }
+            *reinterpret_cast<uint4 *>(&gT[lane * kStrideT + 8 * wave]) =
+                make_uint4(b[0] | b[1] << 16, b[2] | b[3] << 16, b[4] | b[5] << 16, b[6] | b[7] << 16);
         }
         __syncthreads();
 
         // backward, layer 3 .. 0
+#pragma unroll
         for (int l = 3; l >= 0; --l) {
-            const int K = mlp_k(l);
-            const uint16_t *aTl = l == 0 ? xT : (l == 1 ? hT1 : (l == 2 ? hT2 : hT3));
-            const uint16_t *arl = l == 1 ? h1 : (l == 2 ? h2 : h3);
-            // G = bf16(g) row-major [32][64] and transposed [64][40]; bias grad = column sums
-            for (int i = lane; i < 32 * 64; i += 64) {
-                const int r = i >> 6, c = i & 63;
-                const uint16_t b = bf16_bits(zs[r][c]);
-                g[r * kStrideHid + c] = b;
-                gT[c * kStrideT + r] = b;
+            // dA_l = G (32 x 64) . W_l^T (64 x 64)
+            floatx16 da = {};
+            if (l > 0 && wave < 2) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    da = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(g + c32 * kStrideHid + 16 * i + 8 * half),
+                                                                 wb[l > 0 ? l - 1 : 0][i], da, 0, 0, 0);
             }
+            // dW^T tile [32 out][32 in] = G^T (32 samples) . A_l
             {
+                const uint16_t *ga = gT + ((wave >> 1) * 32 + c32) * kStrideT + 8 * half;
+                const uint16_t *ab = actT[l] + ((wave & 1) * 32 + c32) * kStrideT + 8 * half;
+                floatx16 c = {};
+#pragma unroll
+                for (int k0 = 0; k0 < 32; k0 += 16)
+                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(ga + k0), ld8(ab + k0), c, 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    floatx4 *p = reinterpret_cast<floatx4 *>(part + l * 4096 + wave * 1024 + q * 256 + lane * 4);
+                    const floatx4 v = {c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
+                    *p = bi == 0 ? v : *p + v;
+                }
+            }
+            // bias gradient: column sums in row order
+            if (wave == 3) {
                 float s = 0.0f;
-                for (int r = 0; r < 32; ++r) s += zs[r][lane];
-                gsum[lane] = s;
+#pragma unroll
+                for (int r = 0; r < 32; ++r) s += zs[r * kTrainRow + lane];
+                float *p = part + 4 * 4096 + l * 64 + lane;
+                *p = bi == 0 ? s : *p + s;
             }
             __syncthreads();
-            part[mlp_p_b(l) + lane] = (bi == 0 ? 0.0f : part[mlp_p_b(l) + lane]) + gsum[lane];
-            // dW^T [64 out][K in] = G^T (64 x 32 samples) . A_l (32 samples x K):
-            // A operand rows = outputs from gT, B operand columns = inputs from aT
-            for (int mt = 0; mt < 2; ++mt) {
-                floatx16 acc[2];
-#pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-                    floatx16 c = {};
-                    const int r = lane & 31, kh = (lane >> 5) * 8;
-#pragma unroll
-                    for (int k0 = 0; k0 < 32; k0 += 16)
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            ld8(gT + (mt * 32 + r) * kStrideT + k0 + kh), ld8(aTl + (nt * 32 + r) * kStrideT + k0 + kh),
-                            c, 0, 0, 0);
-                    acc[nt] = c;
-                }
-                // element (out o, in i) of dW^T -> master layout W_l[i][o]
-#pragma unroll
-                for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int o = mt * 32 + acc_row(v, lane), in = nt * 32 + (lane & 31);
-                        if (in < K) {
-                            float *p = part + mlp_p_w(l) + in * 64 + o;
-                            *p = (bi == 0 ? 0.0f : *p) + acc[nt][v];
-                        }
-                    }
-            }
             if (l == 0) break;
-            // dA_{l} = G (32 x 64) . W_l^T (64 x K): B column n = input, K dim = outputs,
-            // read from Wk_l [K][64] (input-major), then the ReLU mask of the forward
-            floatx16 da[2];
-            {
-                const int r = lane & 31, kh = (lane >> 5) * 8;
+            if (wave < 2) {
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-                    floatx16 c = {};
+                for (int q = 0; q < 4; ++q) {
+                    const int row = 8 * q + 4 * half;
+                    // the forward's ReLU output (stored, rounded) is > 0 exactly where the gradient passes
+                    const uint2 hv = *reinterpret_cast<const uint2 *>(&actT[l][oc * kStrideT + row]);
+                    const uint32_t h[4] = {hv.x & 0xFFFFu, hv.x >> 16, hv.y & 0xFFFFu, hv.y >> 16};
+                    uint32_t b[4];
 #pragma unroll
-                    for (int k0 = 0; k0 < 64; k0 += 16)
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(g + r * kStrideHid + k0 + kh),
-                                                                    ld8(wk[l] + (nt * 32 + r) * 64 + k0 + kh), c, 0, 0, 0);
-                    da[nt] = c;
+                    for (int j = 0; j < 4; ++j) {
+                        const float gv = (h[j] != 0 && (h[j] & 0x8000u) == 0) ? da[4 * q + j] : 0.0f;
+                        zs[(row + j) * kTrainRow + oc] = gv;
+                        b[j] = bf16_bits(gv);
+                        g[(row + j) * kStrideHid + oc] = (uint16_t)b[j];
+                    }
+                    *reinterpret_cast<uint2 *>(&gT[oc * kStrideT + row]) =
+                        make_uint2(b[0] | b[1] << 16, b[2] | b[3] << 16);
                 }
             }
-            __syncthreads();
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int row = acc_row(v, lane), col = nt * 32 + (lane & 31);
-                    // the forward's ReLU output is > 0 exactly where z > 0
-                    const uint16_t hv = arl[row * kStrideHid + col];
-                    zs[row][col] = (hv != 0 && (hv & 0x8000u) == 0) ? da[nt][v] : 0.0f;
-                }
             __syncthreads();
         }
-        __syncthreads();
     }
-    // per-workgroup loss (lanes 0..31 hold row losses)
-    for (int o = 32; o >= 1; o >>= 1) loss_acc += __shfl_xor(loss_acc, o, 64);
-    if (lane == 0) loss_part[blockIdx.x] = loss_acc;
+    // per-workgroup loss (lanes 0..31 of wave 0 hold row losses)
+    if (wave == 0) {
+        for (int o = 32; o >= 1; o >>= 1) loss_acc += __shfl_xor(loss_acc, o, 64);
+        if (lane == 0) loss_part[blockIdx.x] = loss_acc;
+    }
 }
 
-// Sum the workgroup partials in a fixed order (deterministic) into grad.
-__global__ __launch_bounds__(kBlock) void k_mlp_reduce(const float *__restrict__ partial, int parts,
-                                                       float *__restrict__ grad)
+// One Adam step of master parameter i (Kingma & Ba 2015, bias-corrected), then
+// its bf16 copies Wt (output-major) and Wk (input-major).
+struct AdamStep {
+    float lr, b1, b2, eps, c1, c2;
+};
+__device__ inline void adam_update(const MlpDev &m, int i, float gi, const AdamStep &a)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= kMlpParams) return;
-    float s = 0.0f;
-    for (int p = 0; p < parts; ++p) s += partial[(size_t)p * kMlpParams + i];
-    grad[i] = s;
-}
-
-// Adam (Kingma & Ba 2015, bias-corrected) on the FP32 master parameters, then
-// refresh the bf16 copies Wt (output-major) and Wk (input-major).
-__global__ __launch_bounds__(kBlock) void k_mlp_adam(MlpDev m, const float *__restrict__ grad, float lr, float b1,
-                                                     float b2, float eps, float c1, float c2)
-{
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= kMlpParams) return;
-    const float gi = grad[i];
-    const float mi = b1 * m.adam_m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * m.adam_v[i] + (1.0f - b2) * gi * gi;
+    const float mi = a.b1 * m.adam_m[i] + (1.0f - a.b1) * gi;
+    const float vi = a.b2 * m.adam_v[i] + (1.0f - a.b2) * gi * gi;
     m.adam_m[i] = mi;
     m.adam_v[i] = vi;
-    const float p = m.master[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float p = m.master[i] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
     m.master[i] = p;
-    // scatter to the bf16 copies
-    for (int l = 0; l < 4; ++l) {
-        const int K = mlp_k(l), w0 = mlp_p_w(l), b0 = mlp_p_b(l);
-        if (i >= w0 && i < b0) {
-            const int in = (i - w0) / 64, o = (i - w0) % 64;
-            const uint16_t b = bf16_bits(p);
-            m.wt[mlp_w_off(l) + o * K + in] = b;
-            m.wk[mlp_w_off(l) + in * 64 + o] = b;
-        } else if (i >= b0 && i < b0 + 64) {
-            m.bias[l * 64 + (i - b0)] = p;
+    const int l = i / (64 * 64 + 64), e = i % (64 * 64 + 64);
+    if (e < 64 * 64) {
+        const uint16_t b = bf16_bits(p);
+        m.wt[mlp_w_off(l) + (e & 63) * 64 + (e >> 6)] = b;
+        m.wk[mlp_w_off(l) + e] = b;
+    } else {
+        m.bias[l * 64 + (e - 64 * 64)] = p;
+    }
+}
+
+// Sum the workgroup partials in block order (deterministic), 64 elements per
+// workgroup; the last workgroup sums the losses.  ADAM: the optimiser step of
+// those elements follows in the same lanes (no gradient is stored).
+//
+// Bound by reading the partials (34 MB for 512 blocks): each workgroup's 512
+// lanes keep 256 partials' 64 elements in flight (8 x 16 bytes a lane) and pass
+// them through LDS to one wave, whose lanes add one element each in order
+// while the next 256 partials are on their way.  One lane per element reading
+// the partials itself had 65 workgroups with a few loads in flight: 512 blocks
+// took 119 us, 10 us so (the Adam step included).
+constexpr int kReduceLanes = 512, kReduceElems = 64, kReduceParts = 256;
+static_assert(kMlpParams % kReduceElems == 0, "whole groups of elements");
+
+template <bool ADAM>
+__global__ __launch_bounds__(kReduceLanes) void k_mlp_reduce(const float *__restrict__ partial, int parts,
+                                                             const float *__restrict__ loss_part,
+                                                             float *__restrict__ grad, float *__restrict__ loss,
+                                                             MlpDev m, AdamStep step)
+{
+    __shared__ __attribute__((aligned(16))) float sb[kReduceParts * kReduceElems];
+    const int tid = (int)threadIdx.x;
+    if (blockIdx.x == gridDim.x - 1) {
+        // kBlock lanes, each a strided sum, then a fixed tree
+        if (tid < kBlock) {
+            float a = 0.0f;
+            for (int i = tid; i < parts; i += kBlock) a += loss_part[i];
+            sb[tid] = a;
+        }
+        __syncthreads();
+        for (int w = kBlock / 2; w >= 1; w >>= 1) {
+            if (tid < w) sb[tid] += sb[tid + w];
+            __syncthreads();
+        }
+        if (tid == 0) *loss = sb[0];
+        return;
+    }
+    const int e0 = (int)blockIdx.x * kReduceElems;
+    const int p0 = tid >> 4, e4 = (tid & 15) * 4;
+    constexpr int PER = kReduceParts / (kReduceLanes / 16);
+    floatx4 v[PER];
+    auto load = [&](int base) {
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int p = min(base + p0 + k * (kReduceLanes / 16), parts - 1);
+            v[k] = *reinterpret_cast<const floatx4 *>(partial + (size_t)p * kMlpParams + e0 + e4);
+        }
+    };
+    load(0);
+    float s = 0.0f;
+    for (int base = 0; base < parts; base += kReduceParts) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+            *reinterpret_cast<floatx4 *>(sb + (p0 + k * (kReduceLanes / 16)) * kReduceElems + e4) = v[k];
+        __syncthreads();
+        if (base + kReduceParts < parts) load(base + kReduceParts);
+        if (tid < kReduceElems) {
+            const int n = min(kReduceParts, parts - base);
+#pragma unroll 16
+            for (int p = 0; p < n; ++p) s += sb[p * kReduceElems + tid];
         }
     }
+    if (tid < kReduceElems) {
+        const int i = part_to_master(e0 + tid);
+        if (ADAM) adam_update(m, i, s, step);
+        else grad[i] = s;
+    }
+}
+
+// An Adam step of every parameter with a caller's gradient.
+__global__ __launch_bounds__(kBlock) void k_mlp_adam(MlpDev m, const float *__restrict__ grad, AdamStep step)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < kMlpParams) adam_update(m, i, grad[i], step);
 }
 
 // Refresh the bf16 copies and biases from the master vector (after a load).
@@ -365,28 +497,6 @@ __global__ __launch_bounds__(kBlock) void k_mlp_refresh(MlpDev m)
     }
 }
 
-// Deterministic sum of n floats (one workgroup, fixed order per lane then a
-// fixed tree).
-__global__ __launch_bounds__(kBlock) void k_sum_f32(const float *__restrict__ x, int n, float *__restrict__ out)
-{
-    __shared__ float s[kBlock];
-    float a = 0.0f;
-    for (int i = threadIdx.x; i < n; i += kBlock) a += x[i];
-    s[threadIdx.x] = a;
-    __syncthreads();
-    for (int w = kBlock / 2; w >= 1; w >>= 1) {
-        if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = s[0];
-}
-
-hipError_t launch_sum_f32(const float *x, int n, float *out, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_sum_f32, dim3(1), dim3(kBlock), 0, s, x, n, out);
-    return hipGetLastError();
-}
-
 hipError_t launch_mlp_infer(const MlpDev &m, const float *feats, int n, float *out, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
@@ -400,21 +510,32 @@ hipError_t launch_mlp_infer(const MlpDev &m, const float *feats, int n, float *o
 hipError_t launch_mlp_train(const MlpDev &m, const float *feats, const float *targets, const int *idx, int batch,
                             int nb, float *partial, float *loss_part, int parts, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mlp_train, dim3(parts), dim3(64), 0, s, m, feats, targets, idx, batch, nb, partial, loss_part);
+    hipLaunchKernelGGL(k_mlp_train, dim3(parts), dim3(kBlock), 0, s, m, feats, targets, idx, batch, nb, partial,
+                       loss_part);
     return hipGetLastError();
 }
 
-hipError_t launch_mlp_reduce(const float *partial, int parts, float *grad, hipStream_t s)
+hipError_t launch_mlp_reduce(const float *partial, const float *loss_part, int parts, float *grad, float *loss,
+                             hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpParams + kBlock - 1) / kBlock), dim3(kBlock), 0, s, partial, parts, grad);
+    hipLaunchKernelGGL(k_mlp_reduce<false>, dim3(kMlpParams / kReduceElems + 1), dim3(kReduceLanes), 0, s, partial,
+                       parts, loss_part, grad, loss, MlpDev{}, AdamStep{});
+    return hipGetLastError();
+}
+
+hipError_t launch_mlp_reduce_adam(const MlpDev &m, const float *partial, const float *loss_part, int parts, float *loss,
+                                  float lr, float b1, float b2, float eps, float c1, float c2, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_mlp_reduce<true>, dim3(kMlpParams / kReduceElems + 1), dim3(kReduceLanes), 0, s, partial,
+                       parts, loss_part, (float *)nullptr, loss, m, AdamStep{lr, b1, b2, eps, c1, c2});
     return hipGetLastError();
 }
 
 hipError_t launch_mlp_adam(const MlpDev &m, const float *grad, float lr, float b1, float b2, float eps, float c1,
                            float c2, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m, grad, lr, b1, b2,
-                       eps, c1, c2);
+    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + kBlock - 1) / kBlock), dim3(kBlock), 0, s, m, grad,
+                       AdamStep{lr, b1, b2, eps, c1, c2});
     return hipGetLastError();
 }
 

@@ -470,3 +470,57 @@ def test_gradient_reads_only_its_targets(rc):
             got.append((grad.cpu(), lo.cpu()))
     assert torch.isfinite(got[1][0]).all()
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("n", [1, 32, 33, 8160, 8192, 8193, 16416])
+def test_mlp_gradient_sizes(rc, n):
+    """The gradient at the edges of a 32-sample block and of the reduction's
+    groups of 256 blocks (8160, 8192, 8193 rows: 255, 256, 257 blocks; 16416:
+    two whole groups and one more)."""
+    from oracle import mlp
+    from oracle import surrogate as so
+    params, mean, istd, scale = _net(11)
+    x, t = _rand_io(n, 20 + n)
+    layers = so.params_to_layers(params)
+    z, cache = mlp.forward(layers, (x.astype(np.float64) - mean) * istd, emulate_bf16=True)
+    loss, g4 = mlp.loss_and_grad_out(z, t.astype(np.float64))
+    grads = mlp.backward(layers, cache, g4, emulate_bf16=True)
+    with rc.RadianceCascadeStage(64, 64, levels=3) as st:
+        st.mlp_set(params, mean, istd, scale)
+        grad = torch.empty(rc._abi.MLP_PARAMS, dtype=torch.float32, device="cuda:0")
+        lo = torch.empty(1, dtype=torch.float32, device="cuda:0")
+        st.mlp_gradient(torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda(), grad, lo)
+        gl = so.params_to_layers(grad.cpu().numpy())
+    # fp32 accumulation: (blocks + 64) roundings of 2^-24 at most; and an fp32
+    # sum on the other side of a bf16 rounding boundary moves one of the 192 n
+    # activations by 2^-8 of itself: under 1e-4 of the gradient even for one
+    # activation in 2,000
+    blocks = (n + 31) // 32
+    tol = (blocks + 64) * 2.0 ** -24 + 1e-4
+    assert abs(float(lo.item()) - loss) <= tol * abs(loss)
+    for l in range(4):
+        assert rel_l2(gl[l][0], grads[l][0]) <= tol
+        assert rel_l2(gl[l][1], grads[l][1]) <= tol
+
+
+def test_training_batch_of_several_blocks_per_workgroup(rc):
+    """A batch above 32,768 rows gives each workgroup several blocks: one Adam
+    step of it equals the step taken from the same batch's gradient."""
+    n, lr = 65536 + 4096, 1e-3
+    x, t = _rand_io(n, 6)
+    xd, td = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+    with rc.RadianceCascadeStage(64, 64, levels=3) as st:
+        st.train_surrogate_rows(xd, td.clone(), epochs=1, batch=n, lr=1e-30)
+        net = st.mlp_get()                                    # the initial weights
+        scaled = td * float(np.float32(1.0) / np.float32(net["out_scale"]))
+        st.mlp_set(**net)
+        grad = torch.empty(rc._abi.MLP_PARAMS, dtype=torch.float32, device="cuda:0")
+        lo = torch.empty(1, dtype=torch.float32, device="cuda:0")
+        st.mlp_gradient(xd, scaled, grad, lo)
+        g = grad.cpu().numpy().astype(np.float64)
+        rep = st.train_surrogate_rows(xd, td.clone(), epochs=1, batch=n, lr=lr)
+        after = st.mlp_get()["params"]
+    assert abs(rep["epoch_loss"][0] - float(lo.item())) <= 1e-5 * float(lo.item())
+    # first step: p - lr g / (|g| + eps), insensitive to g's rounding except near g = 0
+    d = np.abs(after - (net["params"] - lr * g / (np.abs(g) + 1e-8)))
+    assert np.mean(d > 1e-2 * lr) < 1e-2 and np.mean(d > 0.5 * lr) < 1e-3
