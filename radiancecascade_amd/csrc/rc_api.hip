@@ -1761,32 +1761,26 @@ static rc_status train_rows(rc_ctx *c, const float *feats, float *targets, size_
     } free_guard{owned};
     hipStream_t s = nullptr;
     double *stats = nullptr;
-    int *idx = nullptr;
+    int *idx = nullptr, *shuffle_head = nullptr, *shuffle_next = nullptr;
     float *partial = nullptr, *loss_part = nullptr, *step_loss = nullptr;
     rc_status st;
     // normalisation: per-input mean and std, one RMS scale for the targets
-    const int parts = 1024;
-    HIP_TRY(c, hipMalloc(&stats, (size_t)parts * 2 * kMlpIn * sizeof(double)));
+    constexpr int kStats = 2 * kMlpIn + 2 * kMlpRad;  // sums and sums of squares of both
+    HIP_TRY(c, hipMalloc(&stats, ((size_t)kColParts * 2 * kMlpIn + kStats) * sizeof(double)));
     owned.push_back(stats);
-    std::vector<double> hs((size_t)parts * 2 * kMlpIn);
+    double *const sums = stats + (size_t)kColParts * 2 * kMlpIn;
+    std::vector<double> hs(kStats);
     std::vector<float> mean(kMlpIn), istd(kMlpIn);
-    HIP_TRY(c, launch_col_stats(feats, N, kMlpIn, stats, parts, s));
-    HIP_TRY(c, hipMemcpy(hs.data(), stats, hs.size() * sizeof(double), hipMemcpyDeviceToHost));
+    HIP_TRY(c, launch_col_stats(feats, N, kMlpIn, stats, sums, s));
+    HIP_TRY(c, launch_col_stats(targets, N, kMlpRad, stats, sums + 2 * kMlpIn, s));
+    HIP_TRY(c, hipMemcpy(hs.data(), sums, hs.size() * sizeof(double), hipMemcpyDeviceToHost));
     for (int j = 0; j < kMlpIn; ++j) {
-        double a = 0.0, b = 0.0;
-        for (int p = 0; p < parts; ++p) {
-            a += hs[(size_t)p * 2 * kMlpIn + j];
-            b += hs[(size_t)p * 2 * kMlpIn + kMlpIn + j];
-        }
-        const double mu = a / (double)N, var = fmax(b / (double)N - mu * mu, 0.0);
+        const double mu = hs[j] / (double)N, var = fmax(hs[kMlpIn + j] / (double)N - mu * mu, 0.0);
         mean[j] = (float)mu;
         istd[j] = (float)(1.0 / fmax(sqrt(var), 1e-3));
     }
-    HIP_TRY(c, launch_col_stats(targets, N, kMlpRad, stats, parts, s));
-    HIP_TRY(c, hipMemcpy(hs.data(), stats, hs.size() * sizeof(double), hipMemcpyDeviceToHost));
     double sq = 0.0;
-    for (int p = 0; p < parts; ++p)
-        for (int j = 0; j < kMlpRad; ++j) sq += hs[(size_t)p * 2 * kMlpRad + kMlpRad + j];
+    for (int j = 0; j < kMlpRad; ++j) sq += hs[2 * kMlpIn + kMlpRad + j];
     const float out_scale = (float)fmax(sqrt(sq / ((double)N * kMlpRad)), 1e-6);
     HIP_TRY(c, launch_scale(targets, N * kMlpRad, 1.0f / out_scale, s));
     HIP_TRY(c, hipDeviceSynchronize());
@@ -1805,13 +1799,16 @@ static rc_status train_rows(rc_ctx *c, const float *feats, float *targets, size_
     if (steps < 1) return fail(c, RC_ERR_INVALID, "rc_surrogate_train: fewer samples than one batch");
     HIP_TRY(c, hipMalloc(&idx, N * sizeof(int)));
     owned.push_back(idx);
+    HIP_TRY(c, hipMalloc(&shuffle_head, N * sizeof(int)));
+    owned.push_back(shuffle_head);
+    HIP_TRY(c, hipMalloc(&shuffle_next, N * sizeof(int)));
+    owned.push_back(shuffle_next);
     HIP_TRY(c, hipMalloc(&partial, (size_t)wgs * kMlpParams * sizeof(float)));
     owned.push_back(partial);
     HIP_TRY(c, hipMalloc(&loss_part, (size_t)wgs * sizeof(float)));
     owned.push_back(loss_part);
     HIP_TRY(c, hipMalloc(&step_loss, steps * sizeof(float)));
     owned.push_back(step_loss);
-    std::vector<int> perm(N);
     std::vector<float> hl(steps);
     uint64_t rs = cfg->seed ^ 0x5DEECE66Dull;
     if (rep) {
@@ -1819,14 +1816,8 @@ static rc_status train_rows(rc_ctx *c, const float *feats, float *targets, size_
         rep->version = RC_ABI_VERSION;
     }
     for (uint32_t e = 0; e < cfg->epochs; ++e) {
-        for (size_t i = 0; i < N; ++i) perm[i] = (int)i;
-        for (size_t i = N - 1; i > 0; --i) {
-            const size_t j = (size_t)(mix64(rs) % (uint64_t)(i + 1));
-            const int t = perm[i];
-            perm[i] = perm[j];
-            perm[j] = t;
-        }
-        HIP_TRY(c, hipMemcpy(idx, perm.data(), N * sizeof(int), hipMemcpyHostToDevice));
+        HIP_TRY(c, launch_shuffle(rs, N, idx, shuffle_head, shuffle_next, s));
+        rs += (uint64_t)(N - 1) * 0x9E3779B97F4A7C15ull;  // the draws it took
         const float lr = cfg->lr * powf(cfg->lr_decay > 0.0f ? cfg->lr_decay : 1.0f, (float)e);
         for (size_t k = 0; k < steps; ++k) {
             HIP_TRY(c, launch_mlp_train(c->mlp, feats, targets, idx + k * batch, batch, nb, partial, loss_part, wgs, s));

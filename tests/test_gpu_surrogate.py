@@ -524,3 +524,43 @@ def test_training_batch_of_several_blocks_per_workgroup(rc):
     # first step: p - lr g / (|g| + eps), insensitive to g's rounding except near g = 0
     d = np.abs(after - (net["params"] - lr * g / (np.abs(g) + 1e-8)))
     assert np.mean(d > 1e-2 * lr) < 1e-2 and np.mean(d > 0.5 * lr) < 1e-3
+
+
+def _fisher_yates(n, state):
+    """0 .. n-1 shuffled by the sequential loop on SplitMix64 draws; the state after it."""
+    m64 = (1 << 64) - 1
+    order = list(range(n))
+    for i in range(n - 1, 0, -1):
+        state = (state + 0x9E3779B97F4A7C15) & m64
+        z = state
+        z = ((z ^ (z >> 30)) * 0xBF58476D1CE4E5B9) & m64
+        z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & m64
+        j = (z ^ (z >> 31)) % (i + 1)
+        order[i], order[j] = order[j], order[i]
+    return order, state
+
+
+@pytest.mark.parametrize("n,batch", [(32, 32), (33, 32), (255, 96), (1000, 32), (66000, 64)])
+def test_training_row_order(rc, n, batch):
+    """The rows each epoch trains on are the head of the sequential
+    Fisher-Yates order.  With a step size too small to move a weight, an
+    epoch's mean loss is that of its floor(n / batch) * batch first rows."""
+    from oracle import mlp
+    from oracle import surrogate as so
+    x, t = _rand_io(n, n)
+    t *= np.exp(np.random.default_rng(n).normal(0.0, 1.5, (n, 1))).astype(np.float32)  # rows of unlike loss
+    with rc.RadianceCascadeStage(64, 64, levels=3) as st:
+        rep = st.train_surrogate_rows(torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda(), epochs=3, batch=batch,
+                                      lr=1e-30, seed=9)
+        net = st.mlp_get()
+    z, _ = mlp.forward(so.params_to_layers(net["params"]),
+                       (x.astype(np.float64) - net["in_mean"]) * net["in_istd"], emulate_bf16=True)
+    rows = ((z[:, :48] - t.astype(np.float64) / net["out_scale"]) ** 2).mean(axis=1)
+    rows = rows + mlp.ERR_WEIGHT * (z[:, 48] - np.log(rows + mlp.ERR_EPS)) ** 2
+    state = 9 ^ 0x5DEECE66D
+    used = n // batch * batch
+    for e in range(3):
+        order, state = _fisher_yates(n, state)
+        want = rows[order[:used]].mean()
+        # bf16 activations on the other side of a rounding boundary, and fp32 sums
+        assert abs(rep["epoch_loss"][e] - want) <= 2e-5 * want, e
