@@ -41,118 +41,113 @@ __device__ inline uint16_t bf16_bits(float f) { return (uint16_t)f32_to_bf16_rne
 
 // LDS row strides (elements) with 8 bf16 of padding: 16-byte aligned rows that
 // do not all start on the same bank.
-constexpr int kStrideIn = kMlpIn + 8;    // 56
-constexpr int kStrideHid = kMlpHid + 8;  // 72
+constexpr int kStrideHid = kMlpHid + 8;
 constexpr int kStrideT = 32 + 8;         // transposed activations [feature][sample]
 
 __device__ inline bf16x8 ld8(const uint16_t *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 
-// acc[nt] = A (32 x K, row stride sa) . B, B column n = nt*32 + (l%32) read as
-// 8 consecutive K elements at b + n*sb + k.
-template <int K>
-__device__ inline void mfma_rows32(const uint16_t *a, int sa, const uint16_t *b, int sb, floatx16 acc[2])
-{
-    const int lane = threadIdx.x & 63, r = lane & 31, kh = (lane >> 5) * 8;
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-        floatx16 c = {};
-#pragma unroll
-        for (int k0 = 0; k0 < K; k0 += 16)
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(a + r * sa + k0 + kh), ld8(b + (nt * 32 + r) * sb + k0 + kh), c,
-                                                        0, 0, 0);
-        acc[nt] = c;
-    }
-}
-
-__device__ inline int acc_row(int v, int lane) { return ((v >> 2) << 3) + ((lane >> 5) << 2) + (v & 3); }
-
-// Forward of one wave's 32 rows.  x: normalised features as bf16 [32][56] in
-// LDS; h: three hidden buffers [32][72]; wt: bf16 Wt_l (LDS or global);
-// bias: FP32.  Returns the output layer's accumulators (+bias) in z[2].
-// hT (optional): transposed copies [64][40] of the inputs of layers 2..4.
-__device__ inline void mlp_forward32(const uint16_t *x, uint16_t *h1, uint16_t *h2, uint16_t *h3,
-                                     const uint16_t *const wt[4], const float *bias, floatx16 z[2],
-                                     uint16_t *hT1 = nullptr, uint16_t *hT2 = nullptr, uint16_t *hT3 = nullptr)
-{
-    const int lane = threadIdx.x & 63;
-    floatx16 acc[2];
-    const uint16_t *in = x;
-    int sin = kStrideIn;
-    uint16_t *outs[3] = {h1, h2, h3};
-    uint16_t *outsT[3] = {hT1, hT2, hT3};
-#pragma unroll
-    for (int l = 0; l < 4; ++l) {
-        if (l == 0) mfma_rows32<kMlpIn>(in, sin, wt[0], kMlpIn, acc);
-        else mfma_rows32<kMlpHid>(in, sin, wt[l], kMlpHid, acc);
-        if (l == 3) {
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                const float bb = bias[3 * 64 + nt * 32 + (lane & 31)];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) z[nt][v] = acc[nt][v] + bb;
-            }
-            break;
-        }
-        __syncthreads();  // previous readers of the output buffer are done (one wave: a no-op barrier)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-            const int col = nt * 32 + (lane & 31);
-            const float bb = bias[l * 64 + col];
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int row = acc_row(v, lane);
-                const uint16_t hv = bf16_bits(fmaxf(acc[nt][v] + bb, 0.0f));
-                outs[l][row * kStrideHid + col] = hv;
-                if (outsT[l]) outsT[l][col * kStrideT + row] = hv;
-            }
-        }
-        __syncthreads();
-        in = outs[l];
-        sin = kStrideHid;
-    }
-}
-
 // ---- inference over a feature matrix -------------------------------------------
 // features [n][64] (already transformed, standardised here) -> z [n][64]
-// fp32.  Each wave takes a 32-row block per iteration; the iteration count is
-// the same for every wave of the workgroup (a wave past the end computes on
-// zero rows and stores nothing), so the barriers are uniform.
-__global__ __launch_bounds__(kBlock) void k_mlp_infer(MlpDev m, const float *__restrict__ feats, int n,
-                                                      float *__restrict__ out)
+// fp32, 32 rows per wave with no exchange between waves.  Each layer is
+// computed transposed, Z^T = W^T . A^T: a lane is one row of the batch (lane %
+// 32), and the accumulators give it 8 groups of 4 consecutive outputs, the
+// lane 32 further on the other 8.  Rounded to bf16 pairs, v_permlane32_swap
+// between the two halves turns them into the next layer's operand, so
+// activations never leave the registers.  The weight fragments are staged in
+// LDS once per workgroup in the order the lanes read them.
+//
+// Bound by the feature and output rows (51 MB for 100,003 rows: 11 us at the
+// rate of a large copy): 16 loads of 16 bytes a wave in flight, 4 waves per
+// SIMD.  100,003 rows: 72.5 us with activations in LDS (2-byte stores, two
+// barriers a layer), 13.4 us so.
+constexpr int kInferLanes = 512;
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // any row address a caller may pass
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
+
+__device__ inline uint32_t bf16_pair(float lo, float hi) { return f32_to_bf16_rne(lo) | (f32_to_bf16_rne(hi) << 16); }
+
+__global__ __launch_bounds__(kInferLanes, 4) void k_mlp_infer(MlpDev m, const float *__restrict__ feats, int n,
+                                                              float *__restrict__ out)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t wt_s[kMlpWt];
-    __shared__ float bias_s[4 * 64], mean_s[kMlpIn], istd_s[kMlpIn];
-    __shared__ __attribute__((aligned(16))) uint16_t buf[4][32 * kStrideIn + 3 * 32 * kStrideHid];
-    for (int i = threadIdx.x; i < kMlpWt; i += kBlock) wt_s[i] = m.wt[i];
-    for (int i = threadIdx.x; i < 4 * 64; i += kBlock) bias_s[i] = m.bias[i];
-    for (int i = threadIdx.x; i < kMlpIn; i += kBlock) {
-        mean_s[i] = m.in_mean[i];
-        istd_s[i] = m.in_istd[i];
+    // fragment (layer, 32-output tile, 16-input chunk): 8 inputs of one output per lane
+    __shared__ uintx4 wf[4][2][4][64];
+    __shared__ __attribute__((aligned(16))) float bias_s[4 * 64], mean_s[kMlpIn], istd_s[kMlpIn];
+    const int lane = threadIdx.x & 63, wave = (int)threadIdx.x >> 6, r = lane & 31, half = lane >> 5;
+    for (int i = threadIdx.x; i < 4 * 2 * 4 * 64; i += kInferLanes) {
+        const int ln = i & 63, k = (i >> 6) & 3, nt = (i >> 8) & 1, l = i >> 9;
+        wf[l][nt][k][ln] = *reinterpret_cast<const uintx4 *>(m.wt + mlp_w_off(l) + (nt * 32 + (ln & 31)) * 64 + 16 * k +
+                                                             8 * (ln >> 5));
+    }
+    if (threadIdx.x < 4 * 64) bias_s[threadIdx.x] = m.bias[threadIdx.x];
+    if (threadIdx.x < kMlpIn) {
+        mean_s[threadIdx.x] = m.in_mean[threadIdx.x];
+        istd_s[threadIdx.x] = m.in_istd[threadIdx.x];
     }
     __syncthreads();
-    const uint16_t *wt[4] = {wt_s, wt_s + 64 * kMlpIn, wt_s + 64 * kMlpIn + 64 * kMlpHid,
-                             wt_s + 64 * kMlpIn + 2 * 64 * kMlpHid};
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    uint16_t *x = buf[wave], *h1 = x + 32 * kStrideIn, *h2 = h1 + 32 * kStrideHid, *h3 = h2 + 32 * kStrideHid;
     const int blocks = (n + 31) / 32;
-    for (int base = blockIdx.x * 4; base < blocks; base += gridDim.x * 4) {
-        const int row0 = (base + wave) * 32;
-        for (int i = lane; i < 32 * kMlpIn; i += 64) {
-            const int r = i / kMlpIn, c = i % kMlpIn;
-            const float v = row0 + r < n ? (feats[(size_t)(row0 + r) * kMlpIn + c] - mean_s[c]) * istd_s[c] : 0.0f;
-            x[r * kStrideIn + c] = bf16_bits(v);
+    for (int b = (int)blockIdx.x * (kInferLanes / 64) + wave; b < blocks; b += (int)gridDim.x * (kInferLanes / 64)) {
+        const size_t row = (size_t)b * 32 + r;
+        // a row past the end computes on the last row's features and stores nothing
+        const float *f = feats + (row < (size_t)n ? row : (size_t)n - 1) * kMlpIn + 8 * half;
+        floatx4 v[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[2 * i] = *reinterpret_cast<const floatx4u *>(f + 16 * i);
+            v[2 * i + 1] = *reinterpret_cast<const floatx4u *>(f + 16 * i + 4);
         }
-        __syncthreads();
-        floatx16 z[2];
-        mlp_forward32(x, h1, h2, h3, wt, bias_s, z);
+        uintx4 x[4];  // the layer's input: 8 features of each 16-feature chunk
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int row = row0 + acc_row(v, lane);
-                if (row < n) out[(size_t)row * kMlpOut + nt * 32 + (lane & 31)] = z[nt][v];
+            for (int h = 0; h < 2; ++h) {
+                const int c = 16 * i + 8 * half + 4 * h;
+                const floatx4 mu = *reinterpret_cast<const floatx4 *>(mean_s + c);
+                const floatx4 sd = *reinterpret_cast<const floatx4 *>(istd_s + c);
+                const floatx4 y = (v[2 * i + h] - mu) * sd;
+                x[i][2 * h] = bf16_pair(y[0], y[1]);
+                x[i][2 * h + 1] = bf16_pair(y[2], y[3]);
             }
-        __syncthreads();
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            asm volatile("" ::: "memory");  // the fragments are read per layer, not held over blocks (128 registers)
+            floatx16 c[2] = {{}, {}};
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    c[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wf[l][nt][i][lane]),
+                                                                    __builtin_bit_cast(bf16x8, x[i]), c[nt], 0, 0, 0);
+            // outputs 32 nt + 8 q + 4 half + {0..3}
+            uint32_t d[2][4][2];
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const floatx4 bb = *reinterpret_cast<const floatx4 *>(bias_s + l * 64 + nt * 32 + 8 * q + 4 * half);
+                    floatx4 y = {c[nt][4 * q], c[nt][4 * q + 1], c[nt][4 * q + 2], c[nt][4 * q + 3]};
+                    y = y + bb;
+                    if (l == 3) {
+                        if (row < (size_t)n)
+                            *reinterpret_cast<floatx4u *>(out + row * kMlpOut + nt * 32 + 8 * q + 4 * half) = y;
+                    } else {
+                        d[nt][q][0] = bf16_pair(fmaxf(y[0], 0.0f), fmaxf(y[1], 0.0f));
+                        d[nt][q][1] = bf16_pair(fmaxf(y[2], 0.0f), fmaxf(y[3], 0.0f));
+                    }
+                }
+            if (l == 3) break;
+            // chunk i of the next input: this half wants group 2 i + half whole,
+            // of which it holds 4 outputs and the other half the other 4
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    const uintx2 sw = __builtin_amdgcn_permlane32_swap(d[i >> 1][2 * (i & 1)][w],
+                                                                       d[i >> 1][2 * (i & 1) + 1][w], false, false);
+                    x[i][w] = sw[0];
+                    x[i][2 + w] = sw[1];
+                }
+        }
     }
 }
 
@@ -605,10 +600,10 @@ hipError_t launch_shuffle(uint64_t state, size_t n, int *order, int *head, int *
 hipError_t launch_mlp_infer(const MlpDev &m, const float *feats, int n, float *out, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    const int blocks32 = (n + 31) / 32;
-    int grid = (blocks32 + 3) / 4;
-    if (grid > 2048) grid = 2048;
-    hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(kBlock), 0, s, m, feats, n, out);
+    // one 32-row block a wave up to 2 workgroups of 8 waves on each of 256 CUs, then several
+    const int blocks = (n + 31) / 32, per = kInferLanes / 64;
+    const int grid = (blocks + per - 1) / per;
+    hipLaunchKernelGGL(k_mlp_infer, dim3(grid < 512 ? grid : 512), dim3(kInferLanes), 0, s, m, feats, n, out);
     return hipGetLastError();
 }
 

@@ -564,3 +564,31 @@ def test_training_row_order(rc, n, batch):
         want = rows[order[:used]].mean()
         # bf16 activations on the other side of a rounding boundary, and fp32 sums
         assert abs(rep["epoch_loss"][e] - want) <= 2e-5 * want, e
+
+
+@pytest.mark.parametrize("n,offset", [(1, 0), (31, 1), (32, 0), (33, 3), (255, 0), (257, 2), (131072, 0), (131105, 1)])
+def test_mlp_forward_sizes(rc, n, offset):
+    """The network alone at the edges of a wave's 32 rows and a workgroup's
+    256, past the largest grid (131,072 rows), on rows that start at any fp32
+    address; nothing is written past the last row."""
+    from oracle import mlp
+    from oracle import surrogate as so
+    params, mean, istd, scale = _net(5)
+    x, _ = _rand_io(n, n)
+    buf = torch.zeros(n * 64 + offset, dtype=torch.float32, device="cuda:0")
+    xd = buf[offset:].view(n, 64)
+    xd.copy_(torch.from_numpy(x))
+    room = torch.full((n * 64 + 64 + offset,), 7.0, dtype=torch.float32, device="cuda:0")
+    out = room[offset:offset + n * 64].view(n, 64)
+    with rc.RadianceCascadeStage(64, 64, levels=3) as st:
+        st.mlp_set(params, mean, istd, scale)
+        st.mlp_forward(xd, out)
+        # the same rows in other lanes, waves and calls: equal bit for bit
+        pieces = torch.empty((n, 64), dtype=torch.float32, device="cuda:0")
+        for i in range(0, n, 1000):
+            st.mlp_forward(torch.from_numpy(x[i:i + 1000]).cuda(), pieces[i:i + 1000])
+        torch.cuda.synchronize()
+    assert torch.equal(out, pieces)
+    z, _ = mlp.forward(so.params_to_layers(params), (x.astype(np.float64) - mean) * istd, emulate_bf16=True)
+    assert rel_l2(out.cpu().numpy(), z) <= MLP_REL_L2
+    assert torch.all(room[offset + n * 64:] == 7.0) and torch.all(room[:offset] == 7.0)
