@@ -65,7 +65,13 @@ typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // any 
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 
-__device__ inline uint32_t bf16_pair(float lo, float hi) { return f32_to_bf16_rne(lo) | (f32_to_bf16_rne(hi) << 16); }
+// Two floats rounded to bf16 (nearest even) in one v_cvt_pk_bf16_f32.
+__device__ inline uint32_t bf16_pair(float lo, float hi)
+{
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){lo, hi}, b2));
+}
 
 __global__ __launch_bounds__(kInferLanes, 4) void k_mlp_infer(MlpDev m, const float *__restrict__ feats, int n,
                                                               float *__restrict__ out)
