@@ -761,3 +761,29 @@ def test_4k_seven_levels_plain_and_learned(rc, oracle):
          f"learned vs plain FP64 {rel_l2(irr_l.cpu().numpy(), irr64):.4f}")
     assert e64 <= REL_L2_TOL_F32
     assert r_l <= 1e-4
+
+
+@pytest.mark.parametrize("W,H,n", [(1, 1, 0), (1, 1, 256), (2, 3, 1), (63, 15, 31), (64, 16, 32), (65, 17, 33),
+                                   (130, 50, 65), (301, 101, 256)])
+def test_raster_tiles_and_chunks(rc, W, H, n):
+    """The G-buffer raster, bit for bit, at the edges of its 64x16-pixel tiles
+    and its chunks of 32 boxes (odd sizes put a column and a row on the optical
+    axis, where a slab's distance is infinite), with boxes a caller may pass
+    beside the scene generator's: around the camera, behind it, inverted,
+    planes through the camera's own, and coplanar (the first one wins)."""
+    from oracle import rco
+    boxes = rc.scene_generate(40 + n, n, min(n, 4))
+    if n >= 31:
+        boxes[3, :6] = [0.2, 0.2, 0.1, 0.9, 0.9, 0.9]      # around the camera
+        boxes[5, :6] = [0.1, 0.1, 0.0, 0.9, 0.9, 0.5]      # ends at the camera's plane
+        boxes[7, :6] = [0.6, 0.7, 0.9, 0.4, 0.2, 0.6]      # inverted
+        boxes[9, :6] = [0.5, 0.5, 0.7, 0.8, 0.8, 0.8]      # planes through the optical axis
+        boxes[11, :6] = boxes[9, :6]                       # coplanar with box 9
+        boxes[30, :6] = [0.45, 0.45, 0.95, 0.55, 0.55, 1.2]  # through the far wall
+    dev = torch.device("cuda:0")
+    depth = torch.empty((H, W), dtype=torch.float32, device=dev)
+    albedo = torch.empty((3, H, W), dtype=torch.float32, device=dev)
+    emis = torch.empty((3, H, W), dtype=torch.float32, device=dev)
+    rc.gbuffer_raster(boxes, W, H, depth, albedo, emis)
+    for got, ref in zip((depth, albedo, emis), rco.raster(boxes, W, H)):
+        assert np.array_equal(got.cpu().numpy().view(np.uint32), ref.view(np.uint32))
