@@ -465,6 +465,7 @@ static rc_status seeds_and_jfa(rc_ctx *c, const float *depth, const float *emiss
     return RC_OK;
 }
 
+// irr == nullptr: the merged levels L-1 .. 1 only, without level 0 and its gather.
 static rc_status run_frame(rc_ctx *c, const float *depth, const float *emissive, float *irr, hipStream_t s,
                            bool quiet = false)
 {
@@ -496,12 +497,14 @@ static rc_status run_frame(rc_ctx *c, const float *depth, const float *emissive,
         c->code_src[i] = split ? 1 : (dbg ? 2 : 0);
     }
     if (top < c->L - 1) c->code_src[c->L - 1] = 1;  // the march stored the top level's codes too
-    tm.begin(RC_STAGE_LEVEL0);
-    LevelArgs a0 = level_args(c, 0, emissive);
-    if (dbg) a0.dbg_codes = c->dbg_codes + c->dbg_code_off[0];
-    HIP_TRY(c, launch_level0_gather(a0, c->storage, irr, dbg ? c->dbg_level0 : nullptr, s));
-    tm.end(RC_STAGE_LEVEL0);
-    c->code_src[0] = dbg ? 2 : 0;
+    if (irr) {
+        tm.begin(RC_STAGE_LEVEL0);
+        LevelArgs a0 = level_args(c, 0, emissive);
+        if (dbg) a0.dbg_codes = c->dbg_codes + c->dbg_code_off[0];
+        HIP_TRY(c, launch_level0_gather(a0, c->storage, irr, dbg ? c->dbg_level0 : nullptr, s));
+        tm.end(RC_STAGE_LEVEL0);
+        c->code_src[0] = dbg ? 2 : 0;
+    }
 
     if (prof) {
         rc_status st = collect_profile(c, s, global_passes);
@@ -828,15 +831,23 @@ static rc_status gen_samples(rc_ctx *c, const float *depth, const float *emissiv
 {
     rc_status st = ensure_surrogate(c);
     if (st != RC_OK) return st;
-    if (!c->scratch_irr) HIP_TRY(c, hipMalloc(&c->scratch_irr, 3 * (size_t)c->W * c->H * sizeof(float)));
-    st = run_frame(c, depth, emissive, c->scratch_irr, s, true);
+    // With the debug copies (level 0's fluence and codes, whole cones) the
+    // frame's irradiance goes to a scratch buffer and the cones are traced
+    // whole; otherwise the rows need neither level 0 nor whole cones.
+    const bool dbg = (c->cfg.flags & RC_FLAG_KEEP_DEBUG) != 0;
+    if (dbg && !c->scratch_irr) HIP_TRY(c, hipMalloc(&c->scratch_irr, 3 * (size_t)c->W * c->H * sizeof(float)));
+    st = run_frame(c, depth, emissive, dbg ? c->scratch_irr : nullptr, s, true);
     if (st != RC_OK) return st;
     HIP_TRY(c, launch_seed_surr(depth, c->depth_conv, emissive, c->occ_bits, c->mip, c->W, c->H, s));
     HIP_TRY(c, launch_mip_top(c->mip, c->flag_count, s));
-    st = launch_cones(c, s);
+    if (dbg) st = launch_cones(c, s);
+    else HIP_TRY(c, launch_cone_pair(cone_args_near(c, false), cone_args_far(c), s));
     if (st != RC_OK) return st;
     SurrSampleArgs a{};
     a.cone = c->cone;
+    a.far = dbg ? nullptr : c->cone_far;
+    a.FX = grid_dim(c->W, 3);
+    a.FY = grid_dim(c->H, 3);
     a.upper = c->level[2];
     a.feats = feats;
     a.targets = targets;

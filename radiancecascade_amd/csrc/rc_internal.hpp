@@ -391,6 +391,8 @@ struct SurrMlpArgs {
 };
 struct SurrSampleArgs {
     const float4 *cone;
+    const float4 *far;      // far-segment cones [FY][FX][16] to append, or nullptr (cone already whole)
+    int FX, FY;
     const void *upper;      // merged level 2 of the plain path (storage texels)
     float *feats;           // [QY*QX][64] per direction log(1 + cone radiance) rgb, T
     float *targets;         // [QY*QX][48] merged level 2 minus cone radiance

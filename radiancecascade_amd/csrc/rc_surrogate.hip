@@ -874,21 +874,38 @@ template <Storage S>
 __global__ __launch_bounds__(kBlock) void k_surr_sample(SurrSampleArgs a)
 {
     using TT = Texel<S>;
-    const int gi = blockIdx.x * kBlock + threadIdx.x;
-    if (gi >= a.QX * a.QY * 16) return;
-    const int k = gi & 15, q = gi >> 4;
-    const typename TT::T *up = (const typename TT::T *)a.upper;
-    const float4 c = a.cone[gi];
-    const float4 u = TT::unpack(up[gi]);
-    float *f = a.feats + (size_t)q * kMlpIn + kMlpFeat * k;
-    float *t = a.targets + (size_t)q * kMlpRad + 3 * k;
-    f[0] = feat_log(c.x);
-    f[1] = feat_log(c.y);
-    f[2] = feat_log(c.z);
-    f[3] = c.w;
-    t[0] = u.x - c.x;
-    t[1] = u.y - c.y;
-    t[2] = u.z - c.z;
+    // a workgroup is 16 probes; its rows of 64 features and 48 targets are
+    // formed in LDS and leave in consecutive stores
+    __shared__ __attribute__((aligned(16))) float fs[16 * kMlpIn], ts[16 * kMlpRad];
+    const int tid = (int)threadIdx.x, n = a.QX * a.QY * 16;
+    const int g0 = (int)blockIdx.x * kBlock, gi = g0 + tid;
+    if (gi < n) {
+        const int k = gi & 15, q = gi >> 4;
+        const typename TT::T *up = (const typename TT::T *)a.upper;
+        float4 c = a.cone[gi];
+        const float4 u = TT::unpack(up[gi]);
+        if (a.far) c = far_append(c, a.far, a.FX, a.FY, q % a.QX, q / a.QX, k);
+        float *f = fs + tid * kMlpFeat;
+        f[0] = feat_log(c.x);
+        f[1] = feat_log(c.y);
+        f[2] = feat_log(c.z);
+        f[3] = c.w;
+        float *t = ts + tid * 3;
+        t[0] = u.x - c.x;
+        t[1] = u.y - c.y;
+        t[2] = u.z - c.z;
+    }
+    __syncthreads();
+    // rows of whole probes (n is a multiple of 16); the caller's buffers may
+    // start at any fp32 address, so the stores are of dwords
+    const int nf = min(kBlock, n - g0) * kMlpFeat, nt = min(kBlock, n - g0) * 3;
+    float *f = a.feats + (size_t)g0 * kMlpFeat, *t = a.targets + (size_t)g0 * 3;
+#pragma unroll
+    for (int i = 0; i < kMlpFeat; ++i)
+        if (tid + i * kBlock < nf) f[tid + i * kBlock] = fs[tid + i * kBlock];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        if (tid + i * kBlock < nt) t[tid + i * kBlock] = ts[tid + i * kBlock];
 }
 
 hipError_t launch_surr_sample(const SurrSampleArgs &a, Storage st, hipStream_t s)
