@@ -1492,6 +1492,12 @@ rc_status rc_gbuffer_raster(const rc_box *boxes, uint32_t n, uint32_t W, uint32_
     if (!dims_ok(W, H) || n > RC_MAX_BOXES) return fail(nullptr, RC_ERR_INVALID, "rc_gbuffer_raster: out of range");
     int ndev = 0;
     if (rc_device_count(&ndev) != RC_OK) return RC_ERR_NO_DEVICE;
+    if (n <= (uint32_t)kRasterArgBoxes) {
+        hipError_t e = launch_raster_args(boxes, (int)n, (int)W, (int)H, depth, albedo, emissive, (hipStream_t)stream);
+        if (e == hipSuccess) e = hipStreamSynchronize((hipStream_t)stream);
+        if (e != hipSuccess) return fail(nullptr, RC_ERR_HIP, std::string("rc_gbuffer_raster: ") + hipGetErrorString(e));
+        return RC_OK;
+    }
     double *dev = nullptr;
     const size_t bytes = (size_t)(n ? n : 1) * sizeof(rc_box);
     hipError_t e = hipMallocAsync((void **)&dev, bytes, (hipStream_t)stream);

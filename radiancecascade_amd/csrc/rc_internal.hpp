@@ -10,6 +10,10 @@ namespace rc {
 
 // ---- scene (rc_scene.hip) ---------------------------------------------------
 void scene_generate(uint64_t seed, int n_boxes, int n_emissive, rc_box *boxes);
+// up to kRasterArgBoxes boxes given by the host, passed as kernel arguments
+constexpr int kRasterArgBoxes = 32;
+hipError_t launch_raster_args(const rc_box *boxes, int n, int W, int H, float *depth, float *albedo, float *emissive,
+                              hipStream_t stream);
 hipError_t launch_raster(const double *boxes_dev, int n, int W, int H, float *depth, float *albedo, float *emissive,
                          hipStream_t stream);
 

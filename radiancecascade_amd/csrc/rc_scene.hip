@@ -67,6 +67,10 @@ void scene_generate(uint64_t seed, int n_boxes, int n_emissive, rc_box *boxes)
 // 1920x1080 with 32 boxes, this form 28 us.
 constexpr int kRasterRows = 16, kRasterChunk = 32;
 
+struct RasterArgs {
+    double box[kRasterArgBoxes * 12];
+};
+
 struct Slab {
     double n, f;  // nearer and farther plane
 };
@@ -82,9 +86,9 @@ __device__ inline void narrow(double &tn, double &tf, const Slab &s)
     if (s.f < tf) tf = s.f;
 }
 
-__global__ __launch_bounds__(kBlock) void k_raster(const double *__restrict__ boxes, int n, int W, int H,
-                                                   float *__restrict__ depth, float *__restrict__ albedo,
-                                                   float *__restrict__ emissive)
+__device__ __forceinline__ void raster_body(const double *__restrict__ boxes, int n, int W, int H,
+                                            float *__restrict__ depth, float *__restrict__ albedo,
+                                            float *__restrict__ emissive)
 {
     __shared__ Slab sx[kRasterChunk][64], sy[kRasterChunk][kRasterRows], sz[kRasterChunk];
     __shared__ int list[RC_MAX_BOXES], list_n;
@@ -187,6 +191,35 @@ __global__ __launch_bounds__(kBlock) void k_raster(const double *__restrict__ bo
             emissive[c * plane + p] = obj[j] < 0 ? 0.0f : (float)boxes[12 * obj[j] + 9 + c];
         }
     }
+}
+
+__global__ __launch_bounds__(kBlock) void k_raster(const double *__restrict__ boxes, int n, int W, int H,
+                                                   float *__restrict__ depth, float *__restrict__ albedo,
+                                                   float *__restrict__ emissive)
+{
+    raster_body(boxes, n, W, H, depth, albedo, emissive);
+}
+
+// A box list short enough to travel with the launch (3 KB of kernel
+// arguments): no device allocation and no copy before the kernel.
+__global__ __launch_bounds__(kBlock) void k_raster_args(RasterArgs r, int n, int W, int H, float *__restrict__ depth,
+                                                        float *__restrict__ albedo, float *__restrict__ emissive)
+{
+    __shared__ double sb[kRasterArgBoxes * 12];
+    for (int i = threadIdx.x; i < n * 12; i += kBlock) sb[i] = r.box[i];
+    __syncthreads();
+    raster_body(sb, n, W, H, depth, albedo, emissive);
+}
+
+hipError_t launch_raster_args(const rc_box *boxes, int n, int W, int H, float *depth, float *albedo, float *emissive,
+                              hipStream_t stream)
+{
+    static_assert(sizeof(rc_box) == 12 * sizeof(double), "a box is 12 doubles");
+    RasterArgs r;
+    for (int i = 0; i < n; ++i) __builtin_memcpy(r.box + 12 * i, boxes + i, sizeof(rc_box));
+    dim3 grid((W + 63) / 64, (H + kRasterRows - 1) / kRasterRows);
+    hipLaunchKernelGGL(k_raster_args, grid, dim3(kBlock), 0, stream, r, n, W, H, depth, albedo, emissive);
+    return hipGetLastError();
 }
 
 hipError_t launch_raster(const double *boxes_dev, int n, int W, int H, float *depth, float *albedo, float *emissive,
