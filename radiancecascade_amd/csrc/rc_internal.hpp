@@ -149,7 +149,7 @@ struct RowJob {
 int occ_blocks(int W, int H);   // 1024-lane workgroups of the occupancy kernel
 int occ_bx(int W);
 int ends_blocks(int W);         // 256-lane workgroups of the band-end kernel
-int edt_row_wmax(int W);        // LDS row capacity of the row kernel (1024 .. 16384)
+int edt_row_wmax(int W);        // LDS row capacity of the row kernel (512 .. 16384)
 hipError_t launch_occ_batch(const BatchLaunch &b, hipStream_t s);
 hipError_t launch_ends_batch(const BatchLaunch &b, hipStream_t s);
 hipError_t launch_rows_batch(const BatchLaunch &b, int wmax, hipStream_t s);  // one workgroup per row

@@ -787,3 +787,45 @@ def test_raster_tiles_and_chunks(rc, W, H, n):
     rc.gbuffer_raster(boxes, W, H, depth, albedo, emis)
     for got, ref in zip((depth, albedo, emis), rco.raster(boxes, W, H)):
         assert np.array_equal(got.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("W,H", [(2, 5), (3, 5), (4, 70), (7, 70), (8, 40), (9, 64), (31, 66), (33, 3), (511, 65),
+                                 (512, 9), (513, 130), (2047, 5), (2048, 66), (4095, 3), (4096, 4), (8191, 2),
+                                 (8192, 3), (96, 16384), (8192, 70)])
+def test_exact_transform_row_blocks(rc, oracle, W, H):
+    """The row transform's blocks of 8 candidates, levels of 1, 2 and 3 bits and
+    lane counts (widths either side of 2^k and of each LDS capacity up to 8192)
+    on occupancy with short and long candidate ranges: a single pixel, two
+    pixels at opposite corners, a column, a row, one site every 8 columns at
+    alternating heights, sparse and dense random pixels, with heights that
+    reach the largest distances."""
+    rng = np.random.default_rng(W * 31 + H)
+    masks = []
+    for kind in ("pixel", "corners", "column", "row", "comb", "sparse", "dense"):
+        m = np.zeros((H, W), bool)
+        if kind == "pixel":
+            m[rng.integers(H), rng.integers(W)] = True
+        elif kind == "corners":
+            m[0, 0] = m[H - 1, W - 1] = True
+        elif kind == "column":
+            m[:, W // 2] = True
+        elif kind == "row":
+            m[H // 3, :] = True
+        elif kind == "comb":
+            m[0, ::8] = True
+            m[H - 1, 4::8] = True
+        else:
+            m = rng.random((H, W)) < (0.002 if kind == "sparse" else 0.4)
+        masks.append(m)
+    d = np.ones((H, W), np.float32)
+    dd = torch.from_numpy(d).cuda()
+    sdf = torch.empty((H, W), dtype=torch.float32, device="cuda:0")
+    irr = torch.empty((3, H, W), dtype=torch.float32, device="cuda:0")
+    with rc.RadianceCascadeStage(W, H, levels=1, debug=True) as st:
+        for m in masks:
+            e = np.zeros((3, H, W), np.float32)
+            e[2] = m
+            st.run_device(dd, torch.from_numpy(e).cuda(), irr)
+            st.debug_sdf(sdf)
+            ref = oracle.sdf_from_d2(oracle.edt_d2(oracle.seed_init(d, e)))
+            assert np.array_equal(sdf.cpu().numpy(), ref)
