@@ -326,6 +326,7 @@ static MarchAllArgs march_all_args(const rc_ctx *c)
     m.sdf = c->sdf;
     m.W = c->W;
     m.H = c->H;
+    int64_t slots = 0;
     for (int i = c->L - 1; i >= 1; --i) {
         MarchLevel &l = m.lev[m.nlev++];
         l.dirs = c->dirs + c->dir_off[i];
@@ -341,12 +342,13 @@ static MarchAllArgs march_all_args(const rc_ctx *c)
         march_level_map(l, c->march_split == 1 ? c->mmap[i] : 0);  // the persistent form is canonical
         l.merged = (i == c->L - 1 && top_merged_in_march(c)) ? c->level[i] : nullptr;
         l.storage = (int)c->storage;
-        const int64_t rays = (int64_t)l.PX * l.PY * l.N, per = (int64_t)kMarchBlock * c->march_m;
-        l.blocks = (int)(((int64_t)l.slots + per - 1) / per);
+        const int64_t rays = (int64_t)l.PX * l.PY * l.N;
+        slots += l.slots;
         l.code_begin = (uint32_t)c->code_off[i];
         l.dir_off = (int)c->dir_off[i];
         m.total_rays += (uint32_t)rays;
     }
+    for (int j = 0; j < m.nlev; ++j) march_level_blocks(m.lev[j], c->spec, c->march_m, slots);
     m.codes_base = c->codes;
     m.dirs_base = c->dirs;
     m.emis4 = c->emis4;

@@ -176,6 +176,7 @@ static hipError_t build_tables(WorkList &w, std::string &err)
     if (w.split && ok) {  // split march: every (view, level >= 1), top level first
         std::vector<MarchJob> j;
         std::vector<int64_t> b;
+        int64_t slots = 0;
         for (int i = w.maxL - 1; i >= 1; --i) {
             for (const WlView &x : w.v) {
                 if (i >= x.L) continue;
@@ -195,11 +196,13 @@ static hipError_t build_tables(WorkList &w, std::string &err)
                 // a view's top level is merged by the march, as in the single-view frame
                 l.merged = (i == x.L - 1 && top_merged(w)) ? (void *)(w.ws + x.level[i]) : nullptr;
                 l.storage = (int)w.st;
-                const int64_t per = (int64_t)kMarchBlock * w.m;
-                l.blocks = (int)(((int64_t)l.slots + per - 1) / per);
+                slots += l.slots;
                 j.push_back(MarchJob{w.ws + x.sdf, (const float4 *)(w.ws + x.emis4), x.W, x.H, l});
-                b.push_back(l.blocks);
             }
+        }
+        for (MarchJob &q : j) {
+            march_level_blocks(q.L, w.spec, w.m, slots);
+            b.push_back(q.L.blocks);
         }
         ok = ok && add_launch(w, blob, WL_MARCH, 0, j, b, kMarchBlock, err);
     }
@@ -326,6 +329,7 @@ hipError_t worklist_create(const rc_view *views, uint32_t n, const uint32_t *lev
     w->ws_bytes = off;
     for (int l = 0; l < RC_MAX_LEVELS; ++l) {
         w->tile[l] = default_level_tile(l, w->maxL);
+        w->mmap[l] = default_march_map(l);
         w->rpt[l] = 2;
     }
     hipError_t e = hipSetDevice(device);

@@ -21,6 +21,8 @@
 // permutations and no LDS.  Before marching, the workgroup stages the upper
 // level's probe neighbourhood for its direction slice in LDS (one global read
 // per texel instead of 16 L2 reads per ray).  Rays that hit skip the merge.
+#include <algorithm>
+
 #include "rc_internal.hpp"
 #include "rc_march.hpp"
 
@@ -46,21 +48,19 @@ __device__ inline Ray ray_begin(float cx, float cy, float dx, float dy, float t0
 }
 
 template <int SPEC>
-__device__ inline void ray_round(Ray &r, __amdgpu_buffer_rsrc_t sdf, int W, int H, float t1)
+__device__ inline void ray_round(Ray &r, const SdfField &f, float t1)
 {
-    float p[SPEC], d[SPEC];
-    int q[SPEC];
-    bool ins[SPEC];
+    float p[SPEC];
+    int ix[SPEC], iy[SPEC];
+    uint32_t c[SPEC];
     p[0] = r.t;
 #pragma unroll
     for (int j = 1; j < SPEC; ++j) p[j] = p[j - 1] + r.guess;
 #pragma unroll
     for (int j = 0; j < SPEC; ++j) {
-        const int ix = floor_i32(fmaf(p[j], r.dx, r.cx));
-        const int iy = floor_i32(fmaf(p[j], r.dy, r.cy));
-        ins[j] = (uint32_t)ix < (uint32_t)W && (uint32_t)iy < (uint32_t)H;
-        q[j] = pixel_index(ix, iy, W);
-        d[j] = sdf_load(sdf, ix, iy, sdf_skip(H));
+        ix[j] = floor_i32(fmaf(p[j], r.dx, r.cx));
+        iy[j] = floor_i32(fmaf(p[j], r.dy, r.cy));
+        c[j] = sdf_code(f, ix[j], iy[j]);
     }
     bool go = true;
 #pragma unroll
@@ -71,19 +71,14 @@ __device__ inline void ray_round(Ray &r, __amdgpu_buffer_rsrc_t sdf, int W, int 
             go = false;
             continue;
         }
-        if (!ins[j]) {
-            r.code = kRayExit;
+        if (c[j] == 0) {
+            const bool ins = (uint32_t)ix[j] < (uint32_t)f.W && (uint32_t)iy[j] < (uint32_t)f.H;
+            r.code = ins ? pixel_index(ix[j], iy[j], f.W) : kRayExit;
             r.alive = false;
             go = false;
             continue;
         }
-        if (d[j] < 0.5f) {
-            r.code = q[j];
-            r.alive = false;
-            go = false;
-            continue;
-        }
-        const float step = march_step(d[j]);
+        const float step = step_of_code(c[j]);
         if (j + 1 < SPEC && step == r.guess) continue;  // p[j+1] == p[j] + step
         r.t = p[j] + step;
         r.guess = step;
@@ -205,7 +200,7 @@ __device__ __forceinline__ void level_body(const LevelArgs &a, int lb)
             cx[j] = ((float)px + 0.5f) * a.spacing;
             cy[j] = ((float)py + 0.5f) * a.spacing;
         }
-        march_rays<RPT>(sdf_rsrc(a.sdf, a.W, a.H), a.W, a.H, cx, cy, dir.x, dir.y, a.t0, a.t1, active, hitq);
+        march_rays<RPT>(sdf_field(a.sdf, a.W, a.H), cx, cy, dir.x, dir.y, a.t0, a.t1, active, hitq);
         if (a.dbg_codes) {
 #pragma unroll
             for (int j = 0; j < RPT; ++j) {
@@ -307,14 +302,13 @@ __device__ __forceinline__ void level0_body(const LevelArgs &a, float *__restric
     const int sx = slot % NX, sy = slot / NX;
     const int px = px0 - 1 + sx, py = py0 - 1 + sy;
     const bool probe = slot < NX * NY && px >= 0 && py >= 0 && px < a.PX && py < a.PY;
-    const __amdgpu_buffer_rsrc_t sdf = sdf_rsrc(a.sdf, a.W, a.H);
-    const int skip = sdf_skip(a.H);
+    const SdfField sdf = sdf_field(a.sdf, a.W, a.H);
     const float cx = ((float)px + 0.5f) * 2.0f, cy = ((float)py + 0.5f) * 2.0f;
     const int ix = 2 * px + 1, iy = 2 * py + 1;  // floor of the probe centre (exact)
     const bool in0 = probe && (uint32_t)ix < (uint32_t)a.W && (uint32_t)iy < (uint32_t)a.H;
     // the first distance sample is issued before the upper level's loads, so
     // the march does not wait for them; they land in LDS after the march
-    const float d0 = in0 ? sdf_load(sdf, ix, iy, skip) : 0.0f;
+    const float d0 = in0 ? sdf_value(sdf_code(sdf, ix, iy)) : 0.0f;
     // the emission of the first sample's pixel (the usual hit) in the same wave
     // of loads, so a hit there needs no dependent load
     const int q0 = in0 ? pixel_index(ix, iy, a.W) : 0;
@@ -355,7 +349,7 @@ __device__ __forceinline__ void level0_body(const LevelArgs &a, float *__restric
                 const int jx = floor_i32(fmaf(t, dir.x, cx)), jy = floor_i32(fmaf(t, dir.y, cy));
                 if (!((uint32_t)jx < (uint32_t)a.W && (uint32_t)jy < (uint32_t)a.H)) {
                     code[k] = kRayExit;
-                } else if (sdf_load(sdf, jx, jy, skip) < 0.5f) {
+                } else if (sdf_code(sdf, jx, jy) == 0) {
                     code[k] = pixel_index(jx, jy, a.W);
                 }
             }
@@ -512,30 +506,33 @@ __device__ inline void decode_ray(const MarchLevel &L, int ray, int &px, int &py
     else if (px >= L.PX) { ++py; px -= L.PX; }
 }
 
-// Split-march slot -> (px, py, k).  Canonical order: the slot is the
-// canonical index.  Wave tiles: slot = T*64 + lane, T = (tile row * ntx +
-// tile column) * slices + slice, lane = (probe in the tile, direction in the
-// slice) with the direction fastest; false for the lanes of a ragged edge
-// tile that fall outside the probe grid.  Rays with nearby start points and
-// directions share a wave, so their march lengths are alike.
-__device__ inline bool decode_slot(const MarchLevel &L, int slot, int &px, int &py, int &k)
+// Split-march slot -> (px, py, k).  Wave tiles: slot = T*64 + lane, T = (tile
+// row * ntx + tile column) * slices + slice, lane = (probe in the tile,
+// direction in the slice) with the direction fastest; false for the lanes of a
+// ragged edge tile that fall outside the probe grid.  Rays with nearby start
+// points and directions share a wave, so their march lengths are alike.
+// Canonical order is the wave tile of one probe x 64 directions, or, for
+// level 1's 16 directions (kd_log = 0), the canonical index itself.  T is
+// wave-uniform, so the tile's row and column are scalar arithmetic: the
+// quotient's estimate by the reciprocal is off by at most one either way.
+__device__ inline bool decode_slot(const MarchLevel &L, int T, int lane, int &px, int &py, int &k)
 {
-    if (!L.map) {
-        decode_ray(L, slot, px, py, k);
-        return true;
+    if (L.map == 0 && L.kd_log == 0) {
+        const int ray = T * 64 + lane;
+        const bool in = ray < (int)L.slots;
+        decode_ray(L, in ? ray : 0, px, py, k);
+        return in;
     }
-    const int lane = slot & 63, T = slot >> 6;
     const int ns_log = L.log2n - L.kd_log;
-    const int slice = T & ((1 << ns_log) - 1);
-    const int tt = T >> ns_log;
-    int ty = (int)((float)tt * L.inv_ntx);
-    int tx = tt - ty * L.ntx;
-    if (tx < 0) { --ty; tx += L.ntx; }
-    else if (tx >= L.ntx) { ++ty; tx -= L.ntx; }
+    const uint32_t tt = (uint32_t)T >> ns_log, ntx = (uint32_t)L.ntx;
+    uint32_t ty = __umulhi(tt, L.rcp_ntx);
+    if (ty * ntx > tt) --ty;
+    if (tt - ty * ntx >= ntx) ++ty;
+    const uint32_t tx = tt - ty * ntx;
     const int pl = lane >> L.kd_log;
-    k = (slice << L.kd_log) | (lane & ((1 << L.kd_log) - 1));
-    px = (tx << L.tx_log) | (pl & ((1 << L.tx_log) - 1));
-    py = (ty << L.ty_log) | (pl >> L.tx_log);
+    k = ((T & ((1 << ns_log) - 1)) << L.kd_log) | (lane & ((1 << L.kd_log) - 1));
+    px = (int)(tx << L.tx_log) | (pl & ((1 << L.tx_log) - 1));
+    py = (int)(ty << L.ty_log) | (pl >> L.tx_log);
     return px < L.PX && py < L.PY;
 }
 
@@ -582,121 +579,126 @@ __device__ inline void merge_top_quad(const MarchLevel &L, const float4 *__restr
     }
 }
 
+// A ray's march from t with SPEC samples per round: sample 0 at t and the
+// next ones where the ray goes if the step stays `guess` (every t is a whole
+// number below 2^24, so t + j guess is exact).  Sample j counts while the step
+// of every one before it was the guess; the last that counts gives the next t.
+// Branch-free, with the interval's end left to the loop: a sample beyond t1
+// can only leave t beyond t1.  Returns where t stopped: at the sample that
+// ended the ray (code 0: off-image or a hit), or at or past t1.
+template <int SPEC>
+__device__ __forceinline__ float march_speculative(const SdfField &f, float cx, float cy, float2 dir, float t,
+                                                   float t1, bool alive)
+{
+    float guess = 1.0f;
+    while (alive) {
+        float p[SPEC], step[SPEC];
+        uint32_t c[SPEC];
+        p[0] = t;
+#pragma unroll
+        for (int j = 1; j < SPEC; ++j) p[j] = p[j - 1] + guess;
+#pragma unroll
+        for (int j = 0; j < SPEC; ++j)
+            c[j] = sdf_code(f, floor_i32(fmaf(p[j], dir.x, cx)), floor_i32(fmaf(p[j], dir.y, cy)));
+#pragma unroll
+        for (int j = 0; j < SPEC; ++j) step[j] = step_of_code(c[j]);
+        float at = p[0], by = step[0];
+        bool same = step[0] == guess;
+#pragma unroll
+        for (int j = 1; j < SPEC; ++j) {
+            at = same ? p[j] : at;
+            by = same ? step[j] : by;
+            same = same && step[j] == guess;
+        }
+        t = at + by;
+        guess = by;
+        alive = by != 0.0f && t < t1;
+    }
+    return t;
+}
+
+// One ray per lane.  The median packet of 64 rays of a 1920x1080 frame ends
+// after 1 to 2 samples and the longest ray takes 339 (791 at 3840x2160), so
+// two things bounded a launch of one packet per wave: handing out 163,200
+// one-wave workgroups takes 36 us alone (4.6 a ns), and a chain of 339
+// dependent samples of 0.17 us each takes as long as the whole launch, 58 us.
+// - A wave takes L.packets packets, a grid's width of waves apart (neighbouring
+//   packets hold rays of like length: 4 in a run gave one wave 4 long ones,
+//   66 us against 60), the next packet's directions read while the present one
+//   marches.
+// - A ray takes its first kMarchPlain samples one per step, in a branch-free
+//   divergent loop on the raw byte code (lanes leave as their rays end), and
+//   the rest kMarchTail at a time: 100 rounds instead of 339 samples for the
+//   longest, in 2,500 of the packets.  Frames of 1920x1080 took 129.1, 128.4,
+//   126.5 and 128.9 us with 8, 12, 16 and 24 plain samples, 151 with no others;
+//   6 and 8 samples a round 126.3 and 128.5.
+// Both with the field's zeros outside the image: march 60 -> 37 us at 1920x1080.
+constexpr int kMarchPlain = 16, kMarchTail = 4;
+template <int SPEC>
+__device__ __forceinline__ void march_packets(const SdfField &f, const MarchLevel &L, int lb,
+                                              const float4 *__restrict__ emis4)
+{
+    const int lane = (int)threadIdx.x;
+    const float t1 = L.t1;
+    const int end = (int)((L.slots + 63) >> 6), nw = L.blocks;
+    const uint32_t kmask = (1u << L.kd_log) - 1, nmask = (uint32_t)L.N - 1;
+    auto direction = [&](int T) -> float2 {
+        const uint32_t k = L.kd_log ? ((uint32_t)T << L.kd_log) | ((uint32_t)lane & kmask)
+                                    : L.map ? (uint32_t)T : (uint32_t)(T * 64 + lane);
+        return L.dirs[k & nmask];
+    };
+    float2 next = direction(lb);
+    for (int T = lb; T < end; T += nw) {
+        const float2 dir = next;
+        next = direction(T + nw);
+        int px, py, k;
+        const bool valid = decode_slot(L, T, lane, px, py, k);
+        const uint32_t at = ((__umul24((uint32_t)py, (uint32_t)L.PX) + (uint32_t)px) << L.log2n) + (uint32_t)k;
+        const float cx = ((float)px + 0.5f) * L.spacing, cy = ((float)py + 0.5f) * L.spacing;
+        float t = L.t0;
+        bool alive = valid && t < t1;
+        if (SPEC == 1) {
+            for (int step = 0; alive && step < kMarchPlain; ++step) {
+                const uint32_t c = sdf_code(f, floor_i32(fmaf(t, dir.x, cx)), floor_i32(fmaf(t, dir.y, cy)));
+                t = t + step_of_code(c);
+                alive = c != 0 && t < t1;
+            }
+        }
+        if (alive) t = march_speculative<SPEC == 1 ? kMarchTail : SPEC>(f, cx, cy, dir, t, t1, true);
+        const int code = ray_code(f, t, t1, dir.x, dir.y, cx, cy);
+        if (valid) L.codes[at] = code;
+        if (L.merged) merge_top_quad(L, emis4, valid, code, at);
+    }
+}
+
 template <int SPEC, int M>
 __device__ __forceinline__ void march_all_body(const uint8_t *sdf_codes, int W, int H, const MarchLevel &L, int lb,
                                                const float4 *__restrict__ emis4)
 {
-    const __amdgpu_buffer_rsrc_t sdf = sdf_rsrc(sdf_codes, W, H);
+    const SdfField f = sdf_field(sdf_codes, W, H);
+    if (M == 1) {
+        march_packets<SPEC>(f, L, lb, emis4);
+        return;
+    }
     const int base = lb * kMarchBlock * M + (int)threadIdx.x;
-    const int total = L.map ? (int)L.slots : L.PX * L.PY * L.N;
+    const int total = (int)L.slots;
 
     int j = 0, ray = base;
     bool valid = false;      // the slot holds a ray of the grid
     uint32_t at = 0;         // its canonical index (where its code goes)
     Ray r;
     auto start = [&]() {
+        const int slot = ray < total ? ray : 0;
         int px, py, k;
-        valid = decode_slot(L, ray < total ? ray : 0, px, py, k) && ray < total;
+        valid = decode_slot(L, slot >> 6, slot & 63, px, py, k) && ray < total;
         at = ((__umul24((uint32_t)py, (uint32_t)L.PX) + (uint32_t)px) << L.log2n) + (uint32_t)k;
         const float2 dir = L.dirs[k];
         r = ray_begin(((float)px + 0.5f) * L.spacing, ((float)py + 0.5f) * L.spacing, dir.x, dir.y, L.t0, L.t1,
                       valid);
     };
-    if (M == 1 && SPEC > 1) {
-        // One ray per lane, SPEC samples per round: the samples of
-        // ray_round<SPEC> (p[0] = t, p[j] = p[j-1] + guess; sample j accepted
-        // while its step equals the guess), with the lanes' paths as masked
-        // updates and the ray's end read from where t stopped, as below: t is
-        // left at the sample that ended the ray (off-image or a hit), or at or
-        // past t1 when the interval ended.
-        int px, py, k;
-        valid = decode_slot(L, ray < total ? ray : 0, px, py, k) && ray < total;
-        at = ((__umul24((uint32_t)py, (uint32_t)L.PX) + (uint32_t)px) << L.log2n) + (uint32_t)k;
-        const float2 dir = L.dirs[k];
-        const float cx = ((float)px + 0.5f) * L.spacing, cy = ((float)py + 0.5f) * L.spacing;
-        const int skip = sdf_skip(H);
-        const float t1 = L.t1;
-        float t = L.t0, guess = 1.0f;
-        bool alive = valid && t < t1;
-        while (alive) {
-            float p[SPEC];
-            uint32_t c[SPEC];
-            bool ins[SPEC];
-            p[0] = t;
-#pragma unroll
-            for (int j = 1; j < SPEC; ++j) p[j] = p[j - 1] + guess;
-#pragma unroll
-            for (int j = 0; j < SPEC; ++j) {
-                const int ix = floor_i32(fmaf(p[j], dir.x, cx)), iy = floor_i32(fmaf(p[j], dir.y, cy));
-                ins[j] = (uint32_t)ix < (uint32_t)W && (uint32_t)iy < (uint32_t)H;
-                c[j] = sdf_code_load(sdf, ix, iy, skip);
-            }
-            bool go = true;
-#pragma unroll
-            for (int j = 0; j < SPEC; ++j) {
-                if (!go) continue;
-                if ((j > 0 && !(p[j] < t1)) || !ins[j] || c[j] == 0) {
-                    // the interval ended at the previous step, or this sample
-                    // left the image or hit: the ray ends at p[j]
-                    t = p[j];
-                    alive = false;
-                    go = false;
-                    continue;
-                }
-                const float step = step_of_code(c[j]);
-                if (j + 1 < SPEC && step == guess) continue;  // p[j+1] == p[j] + step
-                t = p[j] + step;
-                guess = step;
-                alive = t < t1;
-                go = false;
-            }
-        }
-        int code = kRayT1;
-        if (t < t1) {
-            const int ix = floor_i32(fmaf(t, dir.x, cx)), iy = floor_i32(fmaf(t, dir.y, cy));
-            code = ((uint32_t)ix < (uint32_t)W && (uint32_t)iy < (uint32_t)H) ? pixel_index(ix, iy, W) : kRayExit;
-        }
-        if (valid) L.codes[at] = code;
-        if (L.merged) merge_top_quad(L, emis4, valid, code, at);
-        return;
-    }
-    if (M == 1 && SPEC == 1) {
-        // One ray per lane, one sample per step: a branch-free body in a
-        // divergent loop (lanes leave as their rays end) on the raw byte
-        // code.  The samples are those of ray_round<1> -- the same positions,
-        // the same step -- and the ray's end is read from where t stopped: t
-        // advances only on an in-image sample, by 0 on a hit (code 0), so a
-        // ray that ends with t < t1 ended at the sample at t, which is
-        // off-image (exit) or a hit; otherwise it reached t1.
-        int px, py, k;
-        valid = decode_slot(L, ray < total ? ray : 0, px, py, k) && ray < total;
-        at = ((__umul24((uint32_t)py, (uint32_t)L.PX) + (uint32_t)px) << L.log2n) + (uint32_t)k;
-        const float2 dir = L.dirs[k];
-        const float cx = ((float)px + 0.5f) * L.spacing, cy = ((float)py + 0.5f) * L.spacing;
-        const int skip = sdf_skip(H);
-        const float t1 = L.t1;
-        float t = L.t0;
-        bool alive = valid && t < t1;
-        while (alive) {
-            const int ix = floor_i32(fmaf(t, dir.x, cx)), iy = floor_i32(fmaf(t, dir.y, cy));
-            const uint32_t c = sdf_code_load(sdf, ix, iy, skip);
-            const bool ins = (uint32_t)ix < (uint32_t)W && (uint32_t)iy < (uint32_t)H;
-            const float tn = t + step_of_code(c);
-            t = ins ? tn : t;
-            alive = ins && c != 0 && tn < t1;
-        }
-        int code = kRayT1;
-        if (t < t1) {
-            const int ix = floor_i32(fmaf(t, dir.x, cx)), iy = floor_i32(fmaf(t, dir.y, cy));
-            code = ((uint32_t)ix < (uint32_t)W && (uint32_t)iy < (uint32_t)H) ? pixel_index(ix, iy, W) : kRayExit;
-        }
-        if (valid) L.codes[at] = code;
-        if (L.merged) merge_top_quad(L, emis4, valid, code, at);
-        return;
-    }
     start();
     for (;;) {
-        if (r.alive) ray_round<SPEC>(r, sdf, W, H, L.t1);
+        if (r.alive) ray_round<SPEC>(r, f, L.t1);
         if (j < M && !r.alive) {
             if (valid) L.codes[at] = r.code;
             ray += kMarchBlock;
@@ -762,7 +764,7 @@ __global__ __launch_bounds__(kBlock) void k_march_persist(MarchAllArgs a)
         tab_f[threadIdx.x][3] = L.t1;
     }
     __syncthreads();
-    const __amdgpu_buffer_rsrc_t sdf = sdf_rsrc(a.sdf, a.W, a.H);
+    const SdfField f = sdf_field(a.sdf, a.W, a.H);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6));
     const uint32_t np = a.n_packets, nw = a.n_waves;
     // this wave's sequence length (waves past n_waves in the last workgroup have none)
@@ -822,7 +824,7 @@ __global__ __launch_bounds__(kBlock) void k_march_persist(MarchAllArgs a)
             continue;
         }
         if (have) {
-            ray_round<SPEC>(r, sdf, a.W, a.H, t1);
+            ray_round<SPEC>(r, f, t1);
             if (!r.alive) {
                 a.codes_base[out] = r.code;
                 have = false;
@@ -839,9 +841,9 @@ __global__ __launch_bounds__(kBlock) void k_march_persist(MarchAllArgs a)
 __global__ __launch_bounds__(kBlock) void k_ray_decode(MarchLevel l, int64_t *__restrict__ index)
 {
     const int slot = (int)(blockIdx.x * kBlock + threadIdx.x);
-    if (slot >= (l.map ? (int)l.slots : l.PX * l.PY * l.N)) return;
+    if (slot >= (int)l.slots) return;
     int px, py, k;
-    if (decode_slot(l, slot, px, py, k)) index[((int64_t)py * l.PX + px) * l.N + k] = slot;
+    if (decode_slot(l, slot >> 6, slot & 63, px, py, k)) index[((int64_t)py * l.PX + px) * l.N + k] = slot;
 }
 
 template <Storage S>
@@ -1083,27 +1085,38 @@ bool march_map_legal(int level, int map)
 
 void march_level_map(MarchLevel &l, int map)
 {
-    // (tx_log, ty_log, kd_log) of each wave tile
-    static const int tile[kMarchMaps][3] = {{0, 0, 0}, {1, 1, 4}, {2, 2, 2}, {2, 1, 3}, {1, 0, 5}, {3, 3, 0}};
+    // (tx_log, ty_log, kd_log) of each wave tile; canonical order is one probe
+    // x 64 directions where a level has them
+    static const int tile[kMarchMaps][3] = {{0, 0, 6}, {1, 1, 4}, {2, 2, 2}, {2, 1, 3}, {1, 0, 5}, {3, 3, 0}};
     l.map = map;
     l.tx_log = tile[map][0];
     l.ty_log = tile[map][1];
-    l.kd_log = tile[map][2];
-    if (map == 0) {
-        l.ntx = 0;
-        l.inv_ntx = 0.0f;
-        l.slots = (uint32_t)((int64_t)l.PX * l.PY * l.N);
-        return;
-    }
+    l.kd_log = map == 0 && l.log2n < 6 ? 0 : tile[map][2];
     l.ntx = (l.PX + (1 << l.tx_log) - 1) >> l.tx_log;
     const int nty = (l.PY + (1 << l.ty_log) - 1) >> l.ty_log;
-    l.inv_ntx = 1.0f / (float)l.ntx;
-    l.slots = (uint32_t)((int64_t)l.ntx * nty * (l.N >> l.kd_log) * 64);
+    l.rcp_ntx = (uint32_t)std::min<uint64_t>(((1ull << 32) + l.ntx - 1) / l.ntx, 0xFFFFFFFFull);
+    l.slots = map == 0 ? (uint32_t)((int64_t)l.PX * l.PY * l.N)
+                       : (uint32_t)((int64_t)l.ntx * nty * (l.N >> l.kd_log) * 64);
+}
+
+void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64_t launch_slots)
+{
+    l.packets = 1;
+    if (rays_per_lane == 1) {
+        // one more packet a wave per 32,768 packets, so that four times the
+        // 8,192 waves the chip holds are left: with 1, 2, 4 and 8 a frame of
+        // 256x256 took 32.2, 34.1, 38.4 and 48.2 us (4,096 packets), 1283x717
+        // 89.6, 86.5, 87.9, 93.8, 1920x1080 133.1, 126.4, 125.7, 130.0, 3840x2160
+        // 553.9, 517.0, 506.8, 503.2, and 16 views of 9.2 megapixels 900, 828, 792, 772
+        l.packets = (int)std::min<int64_t>(std::max<int64_t>(launch_slots >> 21, 1), 8);
+    }
+    const int64_t per = (int64_t)kMarchBlock * rays_per_lane * l.packets;
+    l.blocks = (int)(((int64_t)l.slots + per - 1) / per);
 }
 
 hipError_t launch_ray_decode(const MarchLevel &l, int64_t *index, hipStream_t s)
 {
-    const int64_t total = l.map ? (int64_t)l.slots : (int64_t)l.PX * l.PY * l.N;
+    const int64_t total = (int64_t)l.slots;
     const unsigned blocks = (unsigned)((total + kBlock - 1) / kBlock);
     if (blocks == 0) return hipSuccess;
     hipLaunchKernelGGL(k_ray_decode, dim3(blocks), dim3(kBlock), 0, s, l, index);

@@ -44,10 +44,14 @@ __host__ __device__ inline int64_t interval_t1(int level) { return (2 * ((1ll <<
 // At 1 byte per pixel the field of a 1920x1080 frame is 2 MB and stays in
 // each XCD's 4 MB L2 while the long rays of the upper levels sample it.  The
 // bytes are stored in vertical strips 16 pixels wide, each padded to a
-// multiple of 8 rows, one row of a strip every 16 bytes: an aligned 128-byte
-// line holds a 16x8-pixel block, so the samples of a ray and of neighbouring
-// rays share lines, and the byte of (x, y) is at x + 16 y + (x >> 4) * skip
-// with skip = 16 * rows - 16 (three instructions per sample in the march).
+// multiple of 8 rows with one at least, one row of a strip every 16 bytes: an
+// aligned 128-byte line holds a 16x8-pixel block, so the samples of a ray and
+// of neighbouring rays share lines, and the byte of (x, y) is at x + 16 y +
+// (x >> 4) * skip with skip = 16 * rows - 16 (three instructions per sample).
+// Row H and the last strip's columns from W on hold 0: with the rows outside
+// the image read as row H, and the columns outside the strips off the range of
+// the buffer, every sample outside the image reads 0 and ends its ray as a hit
+// does, without a test of its own in the march.
 constexpr uint32_t kSdfFar = 255;
 constexpr float kSdfFarValue = 2160.0f;
 __host__ __device__ inline uint32_t sdf_code_of_distance(uint32_t d)  // d = floor of the distance
@@ -66,12 +70,21 @@ __host__ __device__ inline uint32_t isqrt_u32(uint32_t d2)
     while ((uint64_t)(r + 1) * (r + 1) <= d2) ++r;
     return r;
 }
-__host__ __device__ inline int sdf_strips(int W) { return (W + 15) >> 4; }
-__host__ __device__ inline int sdf_rows(int H) { return (H + 7) & ~7; }
-__host__ __device__ inline size_t sdf_elems(int W, int H) { return (size_t)sdf_strips(W) * 16 * (size_t)sdf_rows(H); }
+__host__ __device__ inline int sdf_width(int W) { return (W + 15) & ~15; }
+__host__ __device__ inline int sdf_rows(int H) { return (H + 8) & ~7; }
+__host__ __device__ inline size_t sdf_elems(int W, int H) { return (size_t)sdf_width(W) * (size_t)sdf_rows(H); }
 // the strip-to-strip step less the 16 bytes x itself advances per strip
 __host__ __device__ inline int sdf_skip(int H) { return 16 * sdf_rows(H) - 16; }
 __host__ __device__ inline int sdf_index(int x, int y, int skip) { return x + 16 * y + (x >> 4) * skip; }
+// The code of pixel (x, y), and with the last row and column the zeros beyond them.
+__device__ inline void sdf_store(uint8_t *sdf, int x, int y, int W, int H, uint32_t code)
+{
+    const int skip = sdf_skip(H), end = x == W - 1 ? sdf_width(W) : x + 1;
+    sdf[sdf_index(x, y, skip)] = (uint8_t)code;
+    for (int i = x + 1; i < end; ++i) sdf[sdf_index(i, y, skip)] = 0;
+    if (y == H - 1)
+        for (int i = x; i < end; ++i) sdf[sdf_index(i, H, skip)] = 0;
+}
 
 // ---- storage texels ---------------------------------------------------------
 // fp32: float4.  fp16 / bf16: four 16-bit lanes packed in a uint2 (8 bytes).

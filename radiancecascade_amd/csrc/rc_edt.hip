@@ -427,23 +427,27 @@ __device__ __forceinline__ void edt_row_blocks(const uint64_t *__restrict__ bits
     if (ls == 3) edt_block_level<RL, 3>(hs, key, W, 0);
     else if (ls == 1) edt_block_level<RL, 1>(hs, key, W, 0);
     // the codes of 4 consecutive columns in one store (a strip's row is 16
-    // consecutive bytes; columns past W are its padding)
+    // consecutive bytes), 0 in the last strip's columns past W and in row H
     const uint32_t skip = (uint32_t)sdf_skip(H), row = (uint32_t)y << 4;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         const int x0 = 4 * (tid + k * RL);
-        if (x0 < W) {
+        if (x0 < sdf_width(W)) {
             uint32_t word = 0;
+            if (x0 < W) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t x = (uint32_t)(x0 + i);
-                const uint32_t d2 =
-                    ((uint32_t)(key[key_at(x0) + i] >> 32) >> 3) + (uint32_t)__umul24(x, x) - bias;
-                // sdf_code_of_distance: 128 + (d - 128) / 16 = (d + 1920) / 16, 255 from 2160 on
-                const uint32_t d = block_isqrt(d2), far = min((d + 1920u) >> 4, kSdfFar);
-                word |= (d2 >= empty ? kSdfFar : d < 128u ? d : far) << (8 * i);
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t x = (uint32_t)(x0 + i);
+                    const uint32_t d2 =
+                        ((uint32_t)(key[key_at(x0) + i] >> 32) >> 3) + (uint32_t)__umul24(x, x) - bias;
+                    // sdf_code_of_distance: 128 + (d - 128) / 16 = (d + 1920) / 16, 255 from 2160 on
+                    const uint32_t d = block_isqrt(d2), far = min((d + 1920u) >> 4, kSdfFar);
+                    word |= (x0 + i >= W ? 0 : d2 >= empty ? kSdfFar : d < 128u ? d : far) << (8 * i);
+                }
             }
-            *reinterpret_cast<uint32_t *>(sdf + (__umul24((uint32_t)x0 >> 4, skip) + (uint32_t)x0 + row)) = word;
+            uint32_t *at = reinterpret_cast<uint32_t *>(sdf + (__umul24((uint32_t)x0 >> 4, skip) + (uint32_t)x0 + row));
+            at[0] = word;
+            if (y == H - 1) at[4] = 0;
         }
     }
 }
@@ -554,9 +558,6 @@ __device__ __forceinline__ void edt_row_body(const uint64_t *__restrict__ bits, 
         }
         __syncthreads();
     }
-    // the byte of (x, y) at x + 16 y + (x >> 4) skip (sdf_index) in 32-bit
-    // arithmetic: x >> 4 < 2^10 and skip < 2^18 fit the 24-bit multiplier
-    const uint32_t skip = (uint32_t)sdf_skip(H), row = (uint32_t)y << 4;
     for (int x = tid; x < W; x += RL) {
         const int j = edt_opt(opt, x);
         const uint32_t gj = gs[j];
@@ -565,7 +566,7 @@ __device__ __forceinline__ void edt_row_body(const uint64_t *__restrict__ bits, 
             const int dx = x - j;
             code = sdf_code_of_distance(edt_isqrt((uint32_t)__mul24(dx, dx) + (uint32_t)__umul24(gj, gj)));
         }
-        sdf[__umul24((uint32_t)x >> 4, skip) + (uint32_t)x + row] = (uint8_t)code;
+        sdf_store(sdf, x, y, W, H, code);
     }
 }
 

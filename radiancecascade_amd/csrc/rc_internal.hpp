@@ -211,7 +211,7 @@ struct MarchLevel {
     int PX, PY, N, log2n;
     float inv_px;            // 1/PX in fp32 (probe -> row, corrected)
     float t0, t1, spacing;
-    int blocks;              // workgroups of 256*M ray slots (the march grid is blocks x levels)
+    int blocks;              // one-wave workgroups of 64*M*packets slots (the march grid is blocks x levels)
     uint32_t code_begin;     // first ray of this level in the code buffer (levels 1, 2, ... back to back)
     int dir_off;             // first direction of this level in dirs_base
     // Order of the rays over the lanes (k_march_all only): map 0 = canonical
@@ -220,8 +220,9 @@ struct MarchLevel {
     // kd_log = 6), tiles numbered (tile row, tile column, direction slice)
     // with the slice fastest; `slots` counts the padded tiles' lanes.
     int map, tx_log, ty_log, kd_log, ntx;
-    float inv_ntx;
+    uint32_t rcp_ntx;        // ceil(2^32 / ntx), at most 2^32 - 1 (tile -> row, corrected)
     uint32_t slots;
+    int packets;             // packets of 64 slots a wave marches one after another (one ray per lane)
     // The top level (no upper level) merged by the march itself: each lane
     // quad holds the 4 child directions of one texel, so the march writes
     // A_top = quad mean of (hit ? (E, 0) : (0, 1)) here, in `storage`
@@ -235,9 +236,16 @@ struct MarchLevel {
 // directions, 2 = 4x4 x 4, 3 = 4x2 x 8, 4 = 2x1 x 32, 5 = 8x8 x 1.
 constexpr int kMarchMaps = 6;
 bool march_map_legal(int level, int map);
-// fills map, the wave tile, ntx, inv_ntx and slots of a level (PX, PY, N,
-// log2n set); the caller sizes blocks from slots
+// A work list's default order (a single view's is canonical): 2x1 probes x 32
+// directions, canonical where a level has only 16.  16 views of 9.2 megapixels
+// took 761.7 us in it, 771.5 in canonical order, whose waves fan 64 directions
+// of one probe out; a 3840x2160 frame 506.8 and 538.7 (502.4, 621.7 and 534.9
+// in orders 1, 2 and 3).
+inline int default_march_map(int level) { return num_dirs(level) >= 32 ? 4 : 0; }
+// fills map, the wave tile, ntx, rcp_ntx and slots of a level (PX, PY, N, log2n set)
 void march_level_map(MarchLevel &l, int map);
+// fills packets and blocks of a mapped level; launch_slots = the slots of every level (and view) of its launch
+void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64_t launch_slots);
 struct MarchAllArgs {
     const uint8_t *sdf;
     int W, H, nlev;

@@ -17,45 +17,42 @@ __device__ inline float quad_sum(float v)
 }
 
 // The distance field is read through a buffer resource: the strip index is a
-// 32-bit lane offset (no 64-bit address arithmetic per step), and a lane whose
-// sample is off-image may compute any offset -- the load is range-checked and
-// its value unused.
+// 32-bit lane offset (no 64-bit address arithmetic per step), and a sample off
+// the range of the buffer reads 0.
 constexpr int kBufferDword3 = 0x00020000;  // gfx9-family raw buffer, 32-bit data
 
-__device__ inline __amdgpu_buffer_rsrc_t sdf_rsrc(const uint8_t *sdf, int W, int H)
+struct SdfField {
+    __amdgpu_buffer_rsrc_t rsrc;
+    int W, H, skip;
+};
+
+__device__ inline SdfField sdf_field(const uint8_t *sdf, int W, int H)
 {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(sdf), (short)0, (int)sdf_elems(W, H),
-                                             kBufferDword3);
+    return SdfField{__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(sdf), (short)0, (int)sdf_elems(W, H),
+                                                      kBufferDword3),
+                    W, H, sdf_skip(H)};
+}
+
+// The byte code at (x, y), 0 outside the image: a row outside it becomes row
+// H, whose bytes are 0; in the rows 0 .. H the offset of a column left of the
+// image is negative, of one right of the strips past the buffer, and the
+// columns from W to the strips' end hold 0.  (x >> 4) and skip fit the signed
+// 24-bit multiplier: |x| < 2^18 here, skip < 2^19.  A minimum, a shift, a
+// 24-bit multiply-add and a shift-add.  (A swizzled buffer resource takes row
+// and column without any of them, but a byte gather of 64 lanes then takes 36
+// cycles of a CU's address unit instead of 25, and the march is no faster.)
+__device__ inline uint32_t sdf_code(const SdfField &f, int x, int y)
+{
+    const uint32_t row = min((uint32_t)y, (uint32_t)f.H);
+    const int m = __mul24(x >> 4, f.skip) + x;                   // v_mad_i32_i24
+    uint32_t r;                                                  // (row << 4) + m
+    asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(r) : "v"(row), "v"(m));
+    return __builtin_amdgcn_raw_buffer_load_b8(f.rsrc, (int)r, 0, 0);
 }
 
 // Row-major pixel index q = y*W + x (24-bit multiply: W, y < 2^14) -- the
 // hit code and the emissive index.
 __device__ inline int pixel_index(int x, int y, int W) { return (int)__umul24((uint32_t)y, (uint32_t)W) + x; }
-
-// Byte offset of (x, y) in the strip layout, sdf_index's value for an
-// in-image pixel (x >> 4 < 2^10 and skip < 2^18 fit the 24-bit multiplier):
-// a shift, a 24-bit multiply-add and a shift-add.  For an off-image (x, y)
-// the offset may be anything; the range-checked load is then unused.
-__device__ inline uint32_t sdf_offset(int x, int y, int skip)
-{
-    const uint32_t ux = (uint32_t)x;
-    const uint32_t m = __umul24(ux >> 4, (uint32_t)skip) + ux;  // v_mad_u32_u24
-    uint32_t r;                                                  // (y << 4) + m
-    asm("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(r) : "v"(y), "v"(m));
-    return r;
-}
-
-// Distance load (one byte, decoded).
-__device__ inline float sdf_load(__amdgpu_buffer_rsrc_t r, int x, int y, int skip)
-{
-    return sdf_value(__builtin_amdgcn_raw_buffer_load_b8(r, (int)sdf_offset(x, y, skip), 0, 0));
-}
-
-// The raw byte code at (x, y) (same offset and range check as sdf_load).
-__device__ inline uint32_t sdf_code_load(__amdgpu_buffer_rsrc_t r, int x, int y, int skip)
-{
-    return __builtin_amdgcn_raw_buffer_load_b8(r, (int)sdf_offset(x, y, skip), 0, 0);
-}
 
 // march_step(sdf_value(c)) for a code c >= 1 (c = 0 is a hit and takes no
 // step): sdf_value is c below 128 and 16 c - 1920 from 128 on, and
@@ -83,20 +80,30 @@ __device__ inline float march_step(float d) { return __builtin_amdgcn_fmed3f(d, 
 // Ray codes: >= 0 hit pixel y*W+x, -1 left the image, -2 reached t1.
 constexpr int kRayExit = -1, kRayT1 = -2;
 
+// How a ray ended, from where t stopped: t advances only by a sample's step,
+// which is 0 for code 0, so a ray that ends with t < t1 ended at the sample at
+// t, off-image (exit) or a hit; otherwise it reached t1.
+__device__ inline int ray_code(const SdfField &f, float t, float t1, float dx, float dy, float cx, float cy)
+{
+    int code = kRayT1;
+    if (t < t1) {
+        const int ix = floor_i32(fmaf(t, dx, cx)), iy = floor_i32(fmaf(t, dy, cy));
+        code = ((uint32_t)ix < (uint32_t)f.W && (uint32_t)iy < (uint32_t)f.H) ? pixel_index(ix, iy, f.W) : kRayExit;
+    }
+    return code;
+}
+
 // RPT rays per lane marched in lockstep: each iteration issues the RPT
 // distance-field loads back to back, so a lane keeps RPT independent load
 // chains in flight (the march is a chain of dependent gathers and is bound by
 // their latency, not by bandwidth).  A finished ray's slot keeps issuing a
 // (cached, ignored) load until every ray of the lane is done.  The body is
-// branch-free on the raw byte code: t advances only on an in-image sample,
-// by step_of_code (0 on a hit), so where t stops tells how the ray ended --
-// at t1 if t >= t1, else at the sample at t, off-image (exit) or a hit.  The
-// samples, and so the codes, are those of the one-sample-per-step march.
+// branch-free on the raw byte code.  The samples, and so the codes, are those
+// of the one-sample-per-step march.
 template <int RPT>
-__device__ inline void march_rays(__amdgpu_buffer_rsrc_t sdf, int W, int H, const float *cx, const float *cy,
-                                  float dx, float dy, float t0, float t1, const bool *active, int *code)
+__device__ inline void march_rays(const SdfField &f, const float *cx, const float *cy, float dx, float dy, float t0,
+                                  float t1, const bool *active, int *code)
 {
-    const int skip = sdf_skip(H);
     float t[RPT];
     bool alive[RPT];
     bool any = false;
@@ -108,32 +115,22 @@ __device__ inline void march_rays(__amdgpu_buffer_rsrc_t sdf, int W, int H, cons
     }
     while (any) {
         uint32_t c[RPT];
-        bool ins[RPT];
 #pragma unroll
-        for (int j = 0; j < RPT; ++j) {
-            // positions are finite, so the integer test equals 0 <= x < W, 0 <= y < H
-            const int ix = floor_i32(fmaf(t[j], dx, cx[j]));
-            const int iy = floor_i32(fmaf(t[j], dy, cy[j]));
-            ins[j] = (uint32_t)ix < (uint32_t)W && (uint32_t)iy < (uint32_t)H;
-            c[j] = sdf_code_load(sdf, ix, iy, skip);
-        }
+        for (int j = 0; j < RPT; ++j)
+            c[j] = sdf_code(f, floor_i32(fmaf(t[j], dx, cx[j])), floor_i32(fmaf(t[j], dy, cy[j])));
         any = false;
 #pragma unroll
         for (int j = 0; j < RPT; ++j) {
             const float tn = t[j] + step_of_code(c[j]);
-            if (alive[j] && ins[j]) t[j] = tn;
-            alive[j] = alive[j] && ins[j] && c[j] != 0 && tn < t1;
+            if (RPT == 1 || alive[j]) t[j] = tn;
+            alive[j] = alive[j] && c[j] != 0 && tn < t1;
             any = any || alive[j];
         }
     }
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
         code[j] = kRayT1;
-        if (active[j] && t[j] < t1) {
-            const int ix = floor_i32(fmaf(t[j], dx, cx[j]));
-            const int iy = floor_i32(fmaf(t[j], dy, cy[j]));
-            code[j] = ((uint32_t)ix < (uint32_t)W && (uint32_t)iy < (uint32_t)H) ? pixel_index(ix, iy, W) : kRayExit;
-        }
+        if (active[j]) code[j] = ray_code(f, t[j], t1, dx, dy, cx[j], cy[j]);
     }
 }
 

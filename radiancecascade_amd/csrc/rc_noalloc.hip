@@ -36,7 +36,10 @@ constexpr size_t kNoAllocScratchBytes = 64ull << 20;
 constexpr int kNoAllocMaxLevels = 7;
 constexpr int kNoAllocDirs = 4 * ((1 << (2 * kNoAllocMaxLevels)) - 1) / 3;  // sum of N_i, i < 7
 
-static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
+// The distance field, last in the layout, has rows beyond the image's; those
+// that make it a band of 8 rows more lie past the bytes counted.
+constexpr size_t kNoAllocFieldPad = 8 * RC_MAX_DIM;
+static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes + kNoAllocFieldPad];
 static __device__ __align__(256) float2 scratch_dirs[kNoAllocDirs];
 
 constexpr int kNoAllocMaxDevices = 64;
@@ -62,13 +65,12 @@ static NoAllocLayout noalloc_layout(int W, int H, int L)
     off = align256(off + edt_bits_bytes(W, H));
     m.ends = off;
     off = align256(off + edt_ends_bytes(W, H));
-    m.sdf = off;
-    off = align256(off + sdf_elems(W, H));
     for (int i = 1; i < L; ++i) {
         m.level[i] = off;
         off = align256(off + (size_t)grid_dim(W, i) * grid_dim(H, i) * (num_dirs(i) / 4) * sizeof(float4));
     }
-    m.total = off;
+    m.sdf = off;
+    m.total = align256(off + (size_t)sdf_width(W) * ((H + 7) & ~7));
     return m;
 }
 

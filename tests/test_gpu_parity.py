@@ -475,6 +475,39 @@ def test_every_march_order_is_bit_exact(rc, oracle, W, H, L, seed):
         assert n_checked >= 12 * (L - 1) - 12
 
 
+@pytest.mark.parametrize("sdf", ["exact", "jfa"])
+@pytest.mark.parametrize("W,H", [(15, 7), (16, 8), (17, 9), (33, 24), (64, 65), (255, 40), (16, 300), (8200, 8)])
+def test_rays_leave_the_field_at_every_edge(rc, oracle, W, H, sdf):
+    """The field reads 0 outside the image: widths and heights at, below and
+    above its 16-column strips and 8-row bands, rows over 8192 columns, by
+    both distance transforms and both marches.  Codes equal the oracle's."""
+    _say(f"field edges W={W} H={H} sdf={sdf}")
+    L = 4
+    depth, emis = _device_gbuffer(rc, W, H, 1, 32, 4)
+    d, _, e = oracle.gbuffer(1, W, H, 32, 4)
+    irr32, _ = oracle.run(d, e, L, np.float32, want_levels=True)
+    field = oracle.sdf_from_d2(oracle.edt_d2(oracle.seed_init(d, e)))
+    irr = torch.empty((3, H, W), dtype=torch.float32, device="cuda:0")
+    with rc.RadianceCascadeStage(W, H, levels=L, debug=True) as st:
+        st.set_sdf_mode(sdf)
+        got = torch.empty((H, W), dtype=torch.float32, device="cuda:0")
+        for split in (0, 1, 2):
+            st.set_march(split, 1, 1)
+            st.run_device(depth, emis, irr)
+            st.debug_sdf(got)
+            torch.cuda.synchronize()
+            if not np.array_equal(got.cpu().numpy(), field):
+                assert sdf == "jfa"      # the flood may miss a nearest pixel
+                field = got.cpu().numpy()
+            for i in range(1, L):
+                h = torch.empty(rc.level_rays(W, H, i), dtype=torch.int32, device="cuda:0")
+                st.debug_march(i, h)
+                torch.cuda.synchronize()
+                assert np.array_equal(h.cpu().numpy(), oracle.march_level(field, e, i)[1].ravel()), (split, i)
+            if sdf == "exact":
+                assert np.array_equal(irr.cpu().numpy().view(np.uint32), irr32.view(np.uint32)), split
+
+
 @pytest.mark.parametrize("spec", [1, 2, 4])
 def test_persistent_march_is_bit_exact(rc, oracle, spec):
     """The persistent split march (split 2) stores the same ray codes and
