@@ -1379,6 +1379,7 @@ rc_status rc_autotune(rc_ctx *c, const rc_gbuffer *g, float *irr, uint32_t iters
         LevelArgs a = level_args(c, i, g->emissive);
         a.emis4 = c->emis4;  // as the frame runs them (filled by the frames above)
         if (c->march_split) a.codes = c->codes + c->code_off[i];
+        if (a.codes && a.upper) continue;  // a merge has no tile
         for (int shape = 0; shape < TILE_COUNT; ++shape) {
             for (int rpt : {1, 2, 4}) {
                 if (!tiling_legal(i, shape, rpt)) continue;

@@ -217,7 +217,7 @@ static hipError_t build_tables(WorkList &w, std::string &err)
             a.emis4 = (const float4 *)(w.ws + x.emis4);
             if (w.split) a.codes = (const int *)(w.ws + x.codes[i]);
             j.push_back(a);
-            b.push_back(level_blocks(a.PX, a.PY, a.N, w.tile[i], w.rpt[i]));
+            b.push_back(a.codes && a.upper ? merge_blocks(a.PX, a.PY, a.N) : level_blocks(a.PX, a.PY, a.N, w.tile[i], w.rpt[i]));
         }
         ok = ok && add_launch(w, blob, WL_LEVEL, i, j, b, kBlock, err);
     }
@@ -427,7 +427,10 @@ hipError_t worklist_autotune(WorkList *w, int iters, hipStream_t s, std::string 
             int bshape = x.tile[i], brpt = x.rpt[i];
             for (int shape = 0; shape < TILE_COUNT; ++shape) {
                 if (tile_kd(shape) > num_dirs(i)) continue;
+                const bool merges = x.split && top_merged(x);  // every level's jobs have codes and an upper level
+                if (merges && shape != bshape) continue;
                 for (int r : {1, 2, 4}) {
+                    if (merges && r != brpt) continue;
                     x.tile[i] = shape;
                     x.rpt[i] = r;
                     WL_TRY(build_tables(x, err));

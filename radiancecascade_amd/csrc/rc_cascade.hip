@@ -255,6 +255,132 @@ __global__ __launch_bounds__(kBlock) void k_level(LevelArgs a)
     level_body<TX, TY, KD, RPT, S, UPPER, FROM_CODES>(a, xcd_band(blockIdx.x, gridDim.x));
 }
 
+// The merge of level i from its pre-marched codes, 1 <= i < L - 1.  A lane owns
+// one direction of a 2x2 block of probes (even column and row first), so the
+// four bilinear footprints are 3x3 upper texels, their weights are constants
+// and the footprints' x interpolations are shared by two rows of probes; the
+// texels are read straight from memory, 64 (or 16) consecutive directions a
+// wave, without LDS or a barrier.  A quad of lanes holds the 4 children of the
+// 4 probes' next-lower direction: two exchanges leave lane q with probe q's sum
+// in the order (v0 + v1) + (v2 + v3), and every lane stores one texel.
+// Bound by latency and the hits' gathers: 28 us for the 4 merges of a lit
+// 1920x1080 frame, 45 in the staged form of level_body (190 VALU per 128 rays,
+// here 215 to 235 per 256), 77 and 184 at 3840x2160 in half storage.
+__device__ inline float quad_exchange(float keep, float send, int ctrl_xor)
+{
+    const int o = ctrl_xor == 1 ? __builtin_amdgcn_mov_dpp(__float_as_int(send), 0xB1, 0xF, 0xF, false)
+                                : __builtin_amdgcn_mov_dpp(__float_as_int(send), 0x4E, 0xF, 0xF, false);
+    return keep + __int_as_float(o);
+}
+
+// Workgroups of 4 waves: 4x4 probes x 64 directions, or 8x8 probes x 16 (level 1).
+// GATED: the tile fallback's, nothing when no tile is flagged and only the
+// probes the flagged tiles need.
+template <Storage S, bool NARROW, bool GATED>
+__device__ __forceinline__ void merge_body(const LevelArgs &a, int lb)
+{
+    using TT = Texel<S>;
+    if (GATED && *a.gate == 0) return;
+    const int log2n = 31 - __builtin_clz(a.N);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    const int BX = (a.PX + 1) >> 1, BY = (a.PY + 1) >> 1;
+    int bx, by, k;
+    if (NARROW) {
+        const int gx = (BX + 3) >> 2;
+        bx = (lb % gx) * 4 + (lane >> 4);
+        by = (lb / gx) * 4 + wave;
+        k = lane & 15;
+    } else {
+        const int slices = a.N >> 6, gx = (BX + 1) >> 1;
+        const int tile = lb / slices;
+        bx = (tile % gx) * 2 + (wave & 1);
+        by = (tile / gx) * 2 + (wave >> 1);
+        k = (lb % slices) * 64 + lane;
+    }
+    const int qx = lane & 1, qy = (lane >> 1) & 1;  // the probe whose sum this lane ends with
+    if (by >= BY) return;                           // wave-uniform
+    if (!NARROW && bx >= BX) return;
+    bool store = 2 * bx + qx < a.PX && 2 * by + qy < a.PY;
+    if (GATED) {
+        store = store && a.need[(2 * by + qy) * a.PX + 2 * bx + qx] != 0;
+        if (!__any(store)) return;
+    }
+
+    uint32_t ux[3], uy[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        ux[j] = (uint32_t)min(max(bx - 1 + j, 0), a.UX - 1);
+        uy[j] = __umul24((uint32_t)min(max(by - 1 + j, 0), a.UY - 1), (uint32_t)a.UX);
+    }
+    const typename TT::T *up = (const typename TT::T *)a.upper;
+    int code[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t px = (uint32_t)min(2 * bx + (q & 1), a.PX - 1), py = (uint32_t)min(2 * by + (q >> 1), a.PY - 1);
+        code[q] = a.codes[((__umul24(py, (uint32_t)a.PX) + px) << log2n) + (uint32_t)k];
+    }
+    typename TT::T raw[3][3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) raw[r][c] = up[((uy[r] + ux[c]) << log2n) + (uint32_t)k];
+    // hits take their pixel's emission: the 4 loads in one batch (a miss reads
+    // pixel 0's) in a wave with a hit; each under its own lanes' mask, they wait
+    // for one another
+    float4 e[4] = {};
+    if (__any(max(max(code[0], code[1]), max(code[2], code[3])) >= 0)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) e[q] = a.emis4[(uint32_t)max(code[q], 0)];
+    }
+    float v[4][4];
+    // x interpolation of the 3 rows at the even and the odd column
+    float x[3][2][3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const float4 u0 = TT::unpack(raw[r][0]), u1 = TT::unpack(raw[r][1]), u2 = TT::unpack(raw[r][2]);
+        x[r][0][0] = fmaf(0.75f, u1.x, 0.25f * u0.x);
+        x[r][0][1] = fmaf(0.75f, u1.y, 0.25f * u0.y);
+        x[r][0][2] = fmaf(0.75f, u1.z, 0.25f * u0.z);
+        x[r][1][0] = fmaf(0.25f, u2.x, 0.75f * u1.x);
+        x[r][1][1] = fmaf(0.25f, u2.y, 0.75f * u1.y);
+        x[r][1][2] = fmaf(0.25f, u2.z, 0.75f * u1.z);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int dx = q & 1, dy = q >> 1;
+        const float w1 = dy ? 0.25f : 0.75f, w0 = 1.0f - w1;
+        const bool hit = code[q] >= 0;
+        const float4 h = e[q];
+        v[q][0] = hit ? h.x : fmaf(w1, x[dy + 1][dx][0], w0 * x[dy][dx][0]);
+        v[q][1] = hit ? h.y : fmaf(w1, x[dy + 1][dx][1], w0 * x[dy][dx][1]);
+        v[q][2] = hit ? h.z : fmaf(w1, x[dy + 1][dx][2], w0 * x[dy][dx][2]);
+        v[q][3] = hit ? 0.0f : 1.0f;
+    }
+    float s[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const float lo = quad_exchange(qx ? v[1][c] : v[0][c], qx ? v[0][c] : v[1][c], 1);
+        const float hi = quad_exchange(qx ? v[3][c] : v[2][c], qx ? v[2][c] : v[3][c], 1);
+        s[c] = quad_exchange(qy ? hi : lo, qy ? lo : hi, 2) * 0.25f;
+    }
+    if (store) {
+        const uint32_t p = __umul24((uint32_t)(2 * by + qy), (uint32_t)a.PX) + (uint32_t)(2 * bx + qx);
+        ((typename TT::T *)a.out)[(p << (log2n - 2)) + (uint32_t)(k >> 2)] = TT::pack(make_float4(s[0], s[1], s[2], s[3]));
+    }
+}
+
+template <Storage S, bool NARROW, bool GATED>
+__global__ __launch_bounds__(kBlock) void k_merge(LevelArgs a)
+{
+    merge_body<S, NARROW, GATED>(a, xcd_band(blockIdx.x, gridDim.x));
+}
+
+int merge_blocks(int PX, int PY, int N)
+{
+    const int BX = (PX + 1) >> 1, BY = (PY + 1) >> 1;
+    return N < 64 ? ((BX + 3) >> 2) * ((BY + 3) >> 2) : ((BX + 1) >> 1) * ((BY + 1) >> 1) * (N >> 6);
+}
+
 // One level over a work list of views (each job a view's LevelArgs; the top
 // level of a view has no upper level, so UPPER is taken per job).
 template <int TX, int TY, int KD, int RPT, Storage S, bool FROM_CODES>
@@ -265,8 +391,10 @@ __global__ __launch_bounds__(kBlock) void k_level_batch(const LevelArgs *__restr
     const int j = batch_job(begins, njobs, b);
     const LevelArgs a = jobs[j];
     const int lb = b - begins[j];
-    if (a.upper) level_body<TX, TY, KD, RPT, S, true, FROM_CODES>(a, lb);
-    else level_body<TX, TY, KD, RPT, S, false, FROM_CODES>(a, lb);
+    if (!a.upper) level_body<TX, TY, KD, RPT, S, false, FROM_CODES>(a, lb);
+    else if (!FROM_CODES) level_body<TX, TY, KD, RPT, S, true, false>(a, lb);
+    else if (a.N < 64) merge_body<S, true, false>(a, lb);
+    else merge_body<S, false, false>(a, lb);
 }
 
 // Level 0 (4 directions, interval [0,2)) fused with the gather.  A tile owns
@@ -868,8 +996,7 @@ static void launch_level_shape(const LevelArgs &a, hipStream_t s)
 {
     const int blocks = ((a.PX + TX - 1) / TX) * ((a.PY + TY * RPT - 1) / (TY * RPT)) * (a.N / KD);
     if (a.codes) {
-        if (a.upper) hipLaunchKernelGGL((k_level<TX, TY, KD, RPT, S, true, true>), dim3(blocks), dim3(kBlock), 0, s, a);
-        else hipLaunchKernelGGL((k_level<TX, TY, KD, RPT, S, false, true>), dim3(blocks), dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((k_level<TX, TY, KD, RPT, S, false, true>), dim3(blocks), dim3(kBlock), 0, s, a);
     } else {
         if (a.upper) hipLaunchKernelGGL((k_level<TX, TY, KD, RPT, S, true, false>), dim3(blocks), dim3(kBlock), 0, s, a);
         else hipLaunchKernelGGL((k_level<TX, TY, KD, RPT, S, false, false>), dim3(blocks), dim3(kBlock), 0, s, a);
@@ -894,6 +1021,17 @@ template <Storage S>
 static hipError_t launch_level_st(const LevelArgs &a, int shape, int rpt, hipStream_t s)
 {
     if (tile_kd(shape) > a.N) return hipErrorInvalidValue;
+    if (a.codes && a.upper) {
+        const dim3 grid(merge_blocks(a.PX, a.PY, a.N));
+        if (a.gate) {
+            if (a.N < 64) hipLaunchKernelGGL((k_merge<S, true, true>), grid, dim3(kBlock), 0, s, a);
+            else hipLaunchKernelGGL((k_merge<S, false, true>), grid, dim3(kBlock), 0, s, a);
+        } else {
+            if (a.N < 64) hipLaunchKernelGGL((k_merge<S, true, false>), grid, dim3(kBlock), 0, s, a);
+            else hipLaunchKernelGGL((k_merge<S, false, false>), grid, dim3(kBlock), 0, s, a);
+        }
+        return hipGetLastError();
+    }
     switch (rpt) {
     case 1: return launch_level_rpt<1, S>(a, shape, s);
     case 2: return launch_level_rpt<2, S>(a, shape, s);

@@ -273,6 +273,8 @@ struct Level0Job {
     float *irr;
 };
 int level_blocks(int PX, int PY, int N, int shape, int rays_per_lane);
+// workgroups of a level with codes and an upper level (a merge, whatever the tile)
+int merge_blocks(int PX, int PY, int N);
 // level 0 + gather: a workgroup's tile of kL0TX x kL0TY level-0 probes
 constexpr int kL0TX = 16, kL0TY = 12;
 int level0_blocks(int PX, int PY);

@@ -144,16 +144,19 @@ __device__ inline void near_sdf_block(int blk, const uint64_t *__restrict__ bits
         g[r][j] = (uint8_t)d;
     }
     __syncthreads();
+    const int skip = sdf_skip(H);
     for (int i = threadIdx.x; i < kNearT * kNearT; i += kBlock) {
         const int j = i % kNearT, r = i / kNearT, x = x0 + j, y = y0 + r;
-        if (x >= W || y >= H) continue;
+        if (x >= sdf_width(W) || y >= H) continue;
         int best = kNearR * kNearR + 1;
 #pragma unroll
         for (int dy = -kNearR; dy <= kNearR; ++dy) {
             const int gv = g[r + kNearR + dy][j];
             best = min(best, gv * gv + dy * dy);
         }
-        sdf_store(sdf, x, y, W, H, best <= kNearR * kNearR ? isqrt_u32((uint32_t)best) : kSdfFar);
+        uint8_t *at = sdf + sdf_index(x, y, skip);
+        at[0] = (uint8_t)(x >= W ? 0 : best <= kNearR * kNearR ? isqrt_u32((uint32_t)best) : kSdfFar);
+        if (y == H - 1) at[16] = 0;
     }
 }
 
