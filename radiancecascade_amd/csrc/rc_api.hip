@@ -320,9 +320,13 @@ static bool top_merged_in_march(const rc_ctx *c)
     return c->L > 1 && c->march_split == 1 && c->march_m == 1 && c->mmap[c->L - 1] != 5;
 }
 
-static MarchAllArgs march_all_args(const rc_ctx *c)
+// gated: the tile fallback's march of the probes it needs, one ray per lane
+// with the top level merged, whatever the plain frame's mode.
+static MarchAllArgs march_all_args(const rc_ctx *c, bool gated = false)
 {
     MarchAllArgs m{};
+    const int spec = gated ? 1 : c->spec, rays = gated ? 1 : c->march_m;
+    m.gate = gated ? c->flag_count : nullptr;
     m.sdf = c->sdf;
     m.W = c->W;
     m.H = c->H;
@@ -339,16 +343,19 @@ static MarchAllArgs march_all_args(const rc_ctx *c)
         l.spacing = (float)probe_spacing(i);
         l.log2n = 2 + 2 * i;
         l.inv_px = 1.0f / (float)l.PX;
-        march_level_map(l, c->march_split == 1 ? c->mmap[i] : 0);  // the persistent form is canonical
-        l.merged = (i == c->L - 1 && top_merged_in_march(c)) ? c->level[i] : nullptr;
+        const bool merged = i == c->L - 1 && (gated || top_merged_in_march(c));
+        int map = c->march_split == 1 ? c->mmap[i] : 0;  // the persistent form is canonical
+        if (gated && (map == 0 || (merged && map == 5))) map = default_march_map(i);
+        march_level_map(l, map);
+        l.merged = merged ? c->level[i] : nullptr;
+        l.need = gated ? c->need + c->need_off[i] : nullptr;
         l.storage = (int)c->storage;
-        const int64_t rays = (int64_t)l.PX * l.PY * l.N;
         slots += l.slots;
         l.code_begin = (uint32_t)c->code_off[i];
         l.dir_off = (int)c->dir_off[i];
-        m.total_rays += (uint32_t)rays;
+        m.total_rays += (uint32_t)((int64_t)l.PX * l.PY * l.N);
     }
-    for (int j = 0; j < m.nlev; ++j) march_level_blocks(m.lev[j], c->spec, c->march_m, slots);
+    for (int j = 0; j < m.nlev; ++j) march_level_blocks(m.lev[j], spec, rays, slots);
     m.codes_base = c->codes;
     m.dirs_base = c->dirs;
     m.emis4 = c->emis4;
@@ -688,9 +695,11 @@ static rc_status run_frame_surrogate(rc_ctx *c, const float *depth, const float 
     // Tile fallback (finite threshold): the plain far field for the flagged
     // tiles only, decided on the device.  Every kernel reads the flagged-tile
     // count the network kernel left and does nothing when it is zero; the
-    // masked level kernels compute only the probes the flagged tiles need
-    // (their bilinear neighbourhood at each level up), marched in place on
-    // the whole frame's jump-flood field.
+    // march and the merges compute only the probes the flagged tiles need
+    // (their bilinear neighbourhood at each level up) on the whole frame's
+    // field.  One split march of all levels, as the plain frame's: marched in
+    // place, level by level, each level waited for its own longest ray (153 us
+    // of a 1366x768 frame's 223).
     const bool fallback = c->surr_thr < __builtin_huge_valf();
     if (fallback) {
         tm.begin(RC_STAGE_FALLBACK);
@@ -709,9 +718,11 @@ static rc_status run_frame_surrogate(rc_ctx *c, const float *depth, const float 
         fm.max_tiles = c->surr_tiles;
         fm.need_bytes = c->need_bytes;
         HIP_TRY(c, launch_fallback_masks(fm, s));
-        for (int i = c->L - 1; i >= 2; --i) {
+        HIP_TRY(c, launch_march_all(march_all_args(c, true), 1, 1, s));
+        for (int i = c->L - 2; i >= 2; --i) {
             LevelArgs ai = level_args(c, i, emissive);
             ai.emis4 = c->emis4;
+            ai.codes = c->codes + c->code_off[i];
             ai.gate = c->flag_count;
             ai.need = c->need + c->need_off[i];
             HIP_TRY(c, launch_level(ai, c->storage, c->tile[i], c->rpt[i], s));
@@ -730,10 +741,11 @@ static rc_status run_frame_surrogate(rc_ctx *c, const float *depth, const float 
     HIP_TRY(c, launch_level(a1, c->storage, c->surr_tile1 >= 0 ? c->surr_tile1 : c->tile[1],
                             c->surr_rpt1 >= 0 ? c->surr_rpt1 : c->rpt[1], s));
     if (fallback) {
-        // the flagged tiles' level 1 again, plain: marched on the jump-flood
-        // field and merged from the plain level 2, over the learned one
+        // the flagged tiles' level 1 again, plain: merged from the plain level 2,
+        // over the learned one
         LevelArgs af = level_args(c, 1, emissive);
         af.emis4 = c->emis4;
+        af.codes = c->codes + c->code_off[1];
         af.out = c->surr_a1;
         af.gate = c->flag_count;
         af.need = c->need + c->need_off[1];

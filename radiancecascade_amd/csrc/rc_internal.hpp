@@ -231,12 +231,14 @@ struct MarchLevel {
     // least 4 (every order but 5).
     void *merged;
     int storage;
+    const uint8_t *need;     // gated march: [PY][PX] probes to march; the others' codes are left untouched
 };
 // Wave-tile orders of the split march: 0 canonical, 1 = 2x2 probes x 16
 // directions, 2 = 4x4 x 4, 3 = 4x2 x 8, 4 = 2x1 x 32, 5 = 8x8 x 1.
 constexpr int kMarchMaps = 6;
 bool march_map_legal(int level, int map);
-// A work list's default order (a single view's is canonical): 2x1 probes x 32
+// A work list's default order, and that of the tile fallback's march where no
+// other was chosen (a single view's is canonical): 2x1 probes x 32
 // directions, canonical where a level has only 16.  16 views of 9.2 megapixels
 // took 761.7 us in it, 771.5 in canonical order, whose waves fan 64 directions
 // of one probe out; a 3840x2160 frame 506.8 and 538.7 (502.4, 621.7 and 534.9
@@ -251,6 +253,7 @@ struct MarchAllArgs {
     int W, H, nlev;
     MarchLevel lev[RC_MAX_LEVELS];  // top level first
     const float4 *emis4;     // interleaved emission (a merged level's hits)
+    const int *gate;         // gated march: nothing when *gate == 0, only the probes of `need`; nullptr: all rays
     // persistent form: every ray of every level, in 64-ray packets
     int *codes_base;
     const float2 *dirs_base;

@@ -321,6 +321,45 @@ def test_fallback_of_some_tiles(rc, W, H, L, seed, nb, ne):
     assert r_a1 <= FALLBACK_REL_L2 and r_irr <= FALLBACK_REL_L2
 
 
+@pytest.mark.parametrize("march,order", [((1, 1, 1), 0), ((1, 1, 1), 5), ((0, 1, 1), 0), ((1, 1, 2), 0), ((2, 1, 1), 0)])
+@pytest.mark.parametrize("W,H,L", [(97, 61, 3), (333, 201, 5), (640, 65, 6)])
+def test_fallback_march_of_the_needed_probes(rc, W, H, L, march, order):
+    """The fallback's gated march and merges at odd grids and few levels,
+    whatever the plain frame's march, and with another scene's codes left in
+    the buffer: flagged tiles equal the plain level 1 bit for bit, the others
+    the learned one."""
+    _say(f"[gated march] {W}x{H} L={L} march={march} order={order}")
+    params, mean, istd, scale = _net()
+    irr = torch.empty((3, H, W), device="cuda:0")
+    with rc.RadianceCascadeStage(W, H, levels=L) as plain, rc.RadianceCascadeStage(W, H, levels=L) as st:
+        st.mlp_set(params, mean, istd, scale)
+        st.set_march(*march)
+        st.set_march_order(L - 1, order)
+        a1_p = torch.empty(plain.level_shape(1), device="cuda:0")
+        a1_l, a1_f = torch.empty_like(a1_p), torch.empty_like(a1_p)
+        terr = torch.empty(st.surrogate_shapes()["tiles"], device="cuda:0")
+        for seed in (0, 1):
+            depth, emis = _gbuffer(rc, W, H, seed, 32, 4)
+            plain.run_device(depth, emis, irr)
+            plain.debug_level(1, a1_p)
+            st.set_surrogate(True)
+            st.run_device(depth, emis, irr)
+            st.debug_level(1, a1_l)
+            st.debug_surrogate(tile_err=terr)
+            torch.cuda.synchronize()
+            est = terr.cpu().numpy()
+            thr = float(np.median(est))
+            st.set_surrogate(True, threshold=thr)
+            st.run_device(depth, emis, irr)
+            st.debug_level(1, a1_f)
+            torch.cuda.synchronize()
+            py, px = a1_p.shape[:2]
+            flag = np.repeat(np.repeat(~(est <= thr), 16, axis=0), 16, axis=1)[:py, :px]
+            f, p, l = a1_f.cpu().numpy(), a1_p.cpu().numpy(), a1_l.cpu().numpy()
+            assert np.array_equal(f[flag].view(np.uint32), p[flag].view(np.uint32)), seed
+            assert np.array_equal(f[~flag].view(np.uint32), l[~flag].view(np.uint32)), seed
+
+
 def test_surrogate_graph_replay_matches_direct_launches(rc):
     W, H, L = 240, 160, 5
     depth, emis = _gbuffer(rc, W, H, 9, 8, 2)
