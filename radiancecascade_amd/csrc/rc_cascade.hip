@@ -764,32 +764,72 @@ __device__ __forceinline__ float march_speculative(const SdfField &f, float cx, 
 //   6 and 8 samples a round 126.3 and 128.5.
 // Both with the field's zeros outside the image: march 60 -> 37 us at 1920x1080.
 constexpr int kMarchPlain = 16, kMarchTail = 4;
+//
+// What a packet needs beyond its rays is one wave-uniform tile (row, column,
+// slice) and lane constants: start points and addresses are a scalar part plus
+// a lane part, and the level's fields stay in scalar registers (read from the
+// arguments per packet, one after another, they took a launch without march
+// and stores to 14.7 us at 1920x1080).
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
 template <int SPEC, bool GATED>
-__device__ __forceinline__ void march_packets(const SdfField &f, const MarchLevel &L, int lb,
+__device__ __forceinline__ void march_packets(const SdfField &field, const MarchLevel &L, int lb,
                                               const float4 *__restrict__ emis4)
 {
     const int lane = (int)threadIdx.x;
-    const float t1 = L.t1;
-    const int end = (int)((L.slots + 63) >> 6), nw = L.blocks;
-    const uint32_t kmask = (1u << L.kd_log) - 1, nmask = (uint32_t)L.N - 1;
-    auto direction = [&](int T) -> float2 {
-        const uint32_t k = L.kd_log ? ((uint32_t)T << L.kd_log) | ((uint32_t)lane & kmask)
-                                    : L.map ? (uint32_t)T : (uint32_t)(T * 64 + lane);
-        return L.dirs[k & nmask];
-    };
+    SdfField f = field;
+    f.W = uniform(f.W);
+    f.H = uniform(f.H);
+    f.skip = uniform(f.skip);
+    const int PX = uniform(L.PX), PY = uniform(L.PY), log2n = uniform(L.log2n), nw = uniform(L.blocks);
+    const int end = uniform((int)((L.slots + 63) >> 6)), slots = uniform((int)L.slots);
+    const int tx_log = uniform(L.tx_log), ty_log = uniform(L.ty_log);
+    const int spacing = uniform((int)L.spacing), ntx = uniform(L.ntx), rcp = uniform((int)L.rcp_ntx);
+    const float t0 = __int_as_float(uniform(__float_as_int(L.t0))), t1 = __int_as_float(uniform(__float_as_int(L.t1)));
+    const float2 *dirs = L.dirs;
+    int *codes = L.codes;
+    const bool top = L.merged != nullptr;
+    // level 1 in canonical order: 4 consecutive probes x 16 directions, which may wrap to the next row
+    const bool wrap = L.map == 0 && L.kd_log == 0;
+    const int kd_log = uniform(wrap ? 4 : L.kd_log), ns_log = log2n - kd_log;
+    const int smask = (1 << ns_log) - 1;
+    const int lk = lane & ((1 << kd_log) - 1), pl = lane >> kd_log;
+    const int lx = pl & ((1 << tx_log) - 1), ly = pl >> tx_log;
+    const uint32_t lat = wrap ? (uint32_t)lane : ((__umul24((uint32_t)ly, (uint32_t)PX) + (uint32_t)lx) << log2n) + (uint32_t)lk;
+    auto direction = [&](int T) -> float2 { return (dirs + (wrap ? 0 : (T & smask) << kd_log))[lk]; };
+
     float2 next = direction(lb);
     for (int T = lb; T < end; T += nw) {
         const float2 dir = next;
         next = direction(T + nw);
-        int px, py, k;
-        bool valid = decode_slot(L, T, lane, px, py, k);
+        int px, py;
+        bool valid;
+        uint32_t sat;  // the scalar part of the rays' canonical index
+        if (wrap) {
+            int k;
+            const int ray = T * 64 + lane;
+            valid = ray < slots;
+            decode_ray(L, valid ? ray : 0, px, py, k);
+            sat = (uint32_t)T * 64;
+        } else {
+            const uint32_t tt = (uint32_t)T >> ns_log;
+            uint32_t ty = __umulhi(tt, (uint32_t)rcp);
+            if (ty * (uint32_t)ntx > tt) --ty;
+            if (tt - ty * (uint32_t)ntx >= (uint32_t)ntx) ++ty;
+            const int sx = (int)(tt - ty * (uint32_t)ntx) << tx_log, sy = (int)ty << ty_log;
+            px = sx + lx;
+            py = sy + ly;
+            valid = px < PX && py < PY;
+            sat = ((uint32_t)(sy * PX + sx) << log2n) + (uint32_t)((T & smask) << kd_log);
+        }
         if (GATED) {
-            valid = valid && L.need[py * L.PX + px] != 0;
+            valid = valid && L.need[py * PX + px] != 0;
             if (!__any(valid)) continue;
         }
-        const uint32_t at = ((__umul24((uint32_t)py, (uint32_t)L.PX) + (uint32_t)px) << L.log2n) + (uint32_t)k;
-        const float cx = ((float)px + 0.5f) * L.spacing, cy = ((float)py + 0.5f) * L.spacing;
-        float t = L.t0;
+        // (p + 1/2) spacing, a whole number: spacing is even
+        const float cx = (float)((int)__umul24((uint32_t)px, (uint32_t)spacing) + (spacing >> 1));
+        const float cy = (float)((int)__umul24((uint32_t)py, (uint32_t)spacing) + (spacing >> 1));
+        float t = t0;
         bool alive = valid && t < t1;
         if (SPEC == 1) {
             for (int step = 0; alive && step < kMarchPlain; ++step) {
@@ -800,8 +840,8 @@ __device__ __forceinline__ void march_packets(const SdfField &f, const MarchLeve
         }
         if (alive) t = march_speculative<SPEC == 1 ? kMarchTail : SPEC>(f, cx, cy, dir, t, t1, true);
         const int code = ray_code(f, t, t1, dir.x, dir.y, cx, cy);
-        if (valid) L.codes[at] = code;
-        if (L.merged) merge_top_quad(L, emis4, valid, code, at);
+        if (valid) (codes + sat)[lat] = code;
+        if (top) merge_top_quad(L, emis4, valid, code, sat + lat);
     }
 }
 
@@ -1260,12 +1300,14 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
 {
     l.packets = 1;
     if (rays_per_lane == 1) {
-        // one more packet a wave per 32,768 packets, so that four times the
-        // 8,192 waves the chip holds are left: with 1, 2, 4 and 8 a frame of
-        // 256x256 took 32.2, 34.1, 38.4 and 48.2 us (4,096 packets), 1283x717
-        // 89.6, 86.5, 87.9, 93.8, 1920x1080 133.1, 126.4, 125.7, 130.0, 3840x2160
-        // 553.9, 517.0, 506.8, 503.2, and 16 views of 9.2 megapixels 900, 828, 792, 772
-        l.packets = (int)std::min<int64_t>(std::max<int64_t>(launch_slots >> 21, 1), 8);
+        // few enough packets a wave that several times the 8,192 waves the chip
+        // holds are left: with 1, 2, 4 and 8 a frame of 256x256 (4,096 packets) took
+        // 32.2, 34.1, 38.4 and 48.2 us, 1283x717 (72,000) 89.6, 86.5, 87.9 and 93.8,
+        // one scene of 1920x1080 (163,200) 133.1, 126.4, 125.7 and 130.0 and another
+        // 127.4 with 2 and 138.1 with 4, 3840x2160 (783,000) 553.9, 517.0, 506.8 and
+        // 503.2, 16 views of 9.2 megapixels 900, 828, 792 and 772
+        const int64_t n = launch_slots >> 6;
+        l.packets = n < 48 << 10 ? 1 : n < 192 << 10 ? 2 : n < 512 << 10 ? 4 : 8;
     }
     const int64_t per = (int64_t)kMarchBlock * rays_per_lane * l.packets;
     l.blocks = (int)(((int64_t)l.slots + per - 1) / per);
