@@ -15,7 +15,8 @@
 //            the only form in which level i-1 reads level i.
 //   gather : irradiance(pixel) = bilinear over the level-0 fluence A_0.
 //
-// Work mapping: a workgroup (4 wave64) owns TX x TY probes x KD consecutive
+// Work mapping of a level that marches its own rays (a level marched before by
+// k_march_all is merged by k_merge): a workgroup (4 wave64) owns TX x TY probes x KD consecutive
 // directions, lanes direction-fastest.  The 4 children of a level-(i-1)
 // direction sit in one lane quad, so the reduction is two DPP quad
 // permutations and no LDS.  Before marching, the workgroup stages the upper
@@ -106,22 +107,6 @@ __device__ __forceinline__ void level_body(const LevelArgs &a, int lb)
     const int kk = threadIdx.x % KD, pl = threadIdx.x / KD;
     const int px = px0 + pl % TX, pyb = py0 + pl / TX, k = k0 + kk;
 
-    // the tile fallback: nothing when no tile is flagged; only the probes
-    // the flagged tiles need (a workgroup without one leaves at once)
-    if (a.gate && *a.gate == 0) return;
-    bool needed[RPT];
-#pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        const int py = pyb + j * TY;
-        needed[j] = px < a.PX && py < a.PY && (!a.need || a.need[py * a.PX + px] != 0);
-    }
-    if (a.need) {
-        bool any = false;
-#pragma unroll
-        for (int j = 0; j < RPT; ++j) any = any || needed[j];
-        if (!__syncthreads_or(any)) return;
-    }
-
     // 32-bit indices: a level holds fewer than 2^32 rays (W, H <= 16384), N
     // is a power of two, and probe rows and columns are below 2^24
     const int log2n = 31 - __builtin_clz(a.N);
@@ -130,7 +115,7 @@ __device__ __forceinline__ void level_body(const LevelArgs &a, int lb)
     bool active[RPT];
     int hitq[RPT];
 #pragma unroll
-    for (int j = 0; j < RPT; ++j) active[j] = needed[j];
+    for (int j = 0; j < RPT; ++j) active[j] = px < a.PX && pyb + j * TY < a.PY;
 
     // The upper level's neighbourhood for this direction slice, staged in
     // LDS: UN texels per thread, loaded to registers first.
@@ -175,18 +160,16 @@ __device__ __forceinline__ void level_body(const LevelArgs &a, int lb)
     };
 
     if (FROM_CODES) {
-        // The rays were marched by k_march_all.  Their codes, the staging
-        // loads and the hits' emission gathers are all issued before the
-        // barrier, so the three round trips overlap.
+        // the rays were marched by the split march, which did not merge this,
+        // the top level
+        static_assert(!UPPER || !FROM_CODES, "a level with an upper one is merged from codes by merge_body");
 #pragma unroll
         for (int j = 0; j < RPT; ++j) {
             const int py = min(pyb + j * TY, a.PY - 1);
             hitq[j] = a.codes[((__umul24((uint32_t)py, (uint32_t)a.PX) + (uint32_t)min(px, a.PX - 1)) << log2n) +
                               (uint32_t)k];
         }
-        if (UPPER) stage_loads();
         gather_hits();
-        if (UPPER) stage_stores();
     } else {
         if (UPPER) {
             stage_loads();
@@ -394,7 +377,7 @@ __global__ __launch_bounds__(kBlock) void k_level_batch(const LevelArgs *__restr
     const LevelArgs a = jobs[j];
     const int lb = b - begins[j];
     if (!a.upper) level_body<TX, TY, KD, RPT, S, false, FROM_CODES>(a, lb);
-    else if (!FROM_CODES) level_body<TX, TY, KD, RPT, S, true, false>(a, lb);
+    else if constexpr (!FROM_CODES) level_body<TX, TY, KD, RPT, S, true, false>(a, lb);
     else if (a.N < 64) merge_body<S, true, false>(a, lb);
     else merge_body<S, false, false>(a, lb);
 }
@@ -672,12 +655,10 @@ __device__ inline bool decode_slot(const MarchLevel &L, int T, int lane, int &px
 // levels whose rays are longest start earliest, and the long dependent chains
 // of different levels run concurrently instead of one kernel after another.
 //
-// A workgroup owns 256*M consecutive canonical rays ((py*Px+px)*N+k, so a
-// wave is 64 consecutive directions of one probe, or 64/N whole probes) and
-// lane l marches rays base+l, base+l+256, ... one after another without
-// waiting for the other lanes: when its ray ends it starts the next one in the
-// same loop iteration (march lengths differ by two orders of magnitude, so
-// one-ray-per-lane waves idle most lanes while their longest ray runs).
+// With one ray a lane at a time (M = 1) see march_packets.  Otherwise a
+// workgroup owns 64*M consecutive slots and lane l marches slots base+l,
+// base+l+64, ... one after another without waiting for the other lanes: when
+// its ray ends it starts the next one in the same loop iteration.
 // Blocks go round-robin to the XCDs, which interleaves heavy and light tiles.
 // A_top texel of a lane quad, merged in the march: the level kernel's
 // arithmetic for a level without an upper level (quad sums of the 4 rays,

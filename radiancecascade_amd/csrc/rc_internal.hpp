@@ -200,8 +200,8 @@ struct LevelArgs {
     float t0, t1, spacing;
     const int *codes;        // pre-marched ray codes of this level, or nullptr (march in place)
     int *dbg_codes;          // in-place march: each ray's code also stored here (canonical order), or nullptr
-    const int *gate;         // the kernel does nothing when *gate == 0 (nullptr: always runs)
-    const uint8_t *need;     // [PY][PX] probes to compute (nullptr: all); the others are left untouched
+    const int *gate;         // gated merge: nothing when *gate == 0 (nullptr: not gated)
+    const uint8_t *need;     // gated merge: [PY][PX] probes to compute; the others are left untouched
 };
 
 // k_march_all: every level >= 1 in one launch (level-major, top level first).
