@@ -389,7 +389,7 @@ def batch_leg(rc, torch, args, stream, fps_plain):
 KERNEL_FAMILY = [("k_seed_init", "seed"), ("k_occ_bits", "seed"), ("k_edt_ends", "jfa"), ("k_edt_rows", "jfa"),
                  ("k_jfa_pass", "jfa"), ("k_jfa_tail", "jfa"), ("k_jfa_none", "jfa"),
                  ("k_march_all", "march"), ("k_march_persist", "march"), ("k_level0", "level0"),
-                 ("k_level<", "levels")]
+                 ("k_level<", "levels"), ("k_merge<", "levels")]
 
 
 def _family_of(name):
