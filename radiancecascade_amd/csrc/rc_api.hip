@@ -59,7 +59,7 @@ struct rc_ctx {
     int spec = 1;      // speculation depth of the split march (1, 2, 4)
     int march_m = 1;   // rays per lane, marched back to back (1, 2, 4, 8)
     int *codes = nullptr;
-    float4 *emis4 = nullptr;  // the frame's emission interleaved per pixel (plain path)
+    float4 *emis4 = nullptr;  // the frame's emission interleaved, in 4x2-pixel blocks (plain path)
     size_t code_off[RC_MAX_LEVELS] = {};
     double *norm_ws = nullptr;  // error-norm partials
     float *srgb_table = nullptr;  // composite's 256 sRGB thresholds
@@ -243,7 +243,7 @@ static rc_status allocate(rc_ctx *c, uint32_t W, uint32_t H, uint32_t L)
     const size_t n = (size_t)W * H;
     HIP_TRY_ST(ensure_sdf_buffers(c));
     HIP_TRY(c, hipMalloc(&c->sdf, sdf_elems((int)W, (int)H)));
-    HIP_TRY(c, hipMalloc(&c->emis4, n * sizeof(float4)));
+    HIP_TRY(c, hipMalloc(&c->emis4, emis_texels((int)W, (int)H) * sizeof(float4)));
     const size_t tb = texel_bytes(c->storage);
     for (int i = 1; i < (int)L; ++i) {
         const size_t texels = (size_t)grid_dim(W, i) * grid_dim(H, i) * (num_dirs(i) / 4);

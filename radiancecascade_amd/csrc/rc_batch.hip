@@ -315,7 +315,7 @@ hipError_t worklist_create(const rc_view *views, uint32_t n, const uint32_t *lev
         x.sdf = off;
         off = align256(off + sdf_elems(x.W, x.H));
         x.emis4 = off;
-        off = align256(off + 16 * px);
+        off = align256(off + 16 * emis_texels(x.W, x.H));
         for (int l = 1; l < x.L; ++l) {
             const size_t probes = (size_t)grid_dim(x.W, l) * grid_dim(x.H, l);
             x.codes[l] = off;

@@ -150,7 +150,7 @@ __device__ __forceinline__ void level_body(const LevelArgs &a, int lb)
             if (active[j] && hitq[j] >= 0) {
                 const uint32_t q = (uint32_t)hitq[j];
                 if (a.emis4) {
-                    const float4 e = a.emis4[q];
+                    const float4 e = a.emis4[emis_index_of(q, a.W, emis_rcp(a.W))];
                     ev[j] = make_float3(e.x, e.y, e.z);
                 } else {
                     ev[j] = make_float3(a.emissive[q], a.emissive[plane + q], a.emissive[2 * plane + q]);
@@ -246,9 +246,10 @@ __global__ __launch_bounds__(kBlock) void k_level(LevelArgs a)
 // wave, without LDS or a barrier.  A quad of lanes holds the 4 children of the
 // 4 probes' next-lower direction: two exchanges leave lane q with probe q's sum
 // in the order (v0 + v1) + (v2 + v3), and every lane stores one texel.
-// Bound by latency and the hits' gathers: 28 us for the 4 merges of a lit
-// 1920x1080 frame, 45 in the staged form of level_body (190 VALU per 128 rays,
-// here 215 to 235 per 256), 77 and 184 at 3840x2160 in half storage.
+// Bound by latency and the hits' gathers: 24 us for the 4 merges of a lit
+// 1920x1080 frame (28 with the emission row by row), 45 in the staged form of
+// level_body (190 VALU per 128 rays, here 215 to 235 per 256 and 56 more in a
+// wave with a hit), 63 and 184 at 3840x2160 in half storage.
 __device__ inline float quad_exchange(float keep, float send, int ctrl_xor)
 {
     const int o = ctrl_xor == 1 ? __builtin_amdgcn_mov_dpp(__float_as_int(send), 0xB1, 0xF, 0xF, false)
@@ -314,8 +315,9 @@ __device__ __forceinline__ void merge_body(const LevelArgs &a, int lb)
     // for one another
     float4 e[4] = {};
     if (__any(max(max(code[0], code[1]), max(code[2], code[3])) >= 0)) {
+        const float rcp = emis_rcp(a.W);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) e[q] = a.emis4[(uint32_t)max(code[q], 0)];
+        for (int q = 0; q < 4; ++q) e[q] = a.emis4[emis_index_of((uint32_t)max(code[q], 0), a.W, rcp)];
     }
     float v[4][4];
     // x interpolation of the 3 rows at the even and the odd column
@@ -663,13 +665,13 @@ __device__ inline bool decode_slot(const MarchLevel &L, int T, int lane, int &px
 // A_top texel of a lane quad, merged in the march: the level kernel's
 // arithmetic for a level without an upper level (quad sums of the 4 rays,
 // times 1/4), stored by the quad's first lane.
-__device__ inline void merge_top_quad(const MarchLevel &L, const float4 *__restrict__ emis4, bool valid, int code,
+__device__ inline void merge_top_quad(const MarchLevel &L, const float4 *__restrict__ emis4, int W, bool valid, int code,
                                       uint32_t at)
 {
     float r = 0.f, g = 0.f, b = 0.f, al = 0.f;
     if (valid) {
         if (code >= 0) {
-            const float4 e = emis4[code];
+            const float4 e = emis4[emis_index_of((uint32_t)code, W, emis_rcp(W))];
             r = e.x;
             g = e.y;
             b = e.z;
@@ -822,7 +824,7 @@ __device__ __forceinline__ void march_packets(const SdfField &field, const March
         if (alive) t = march_speculative<SPEC == 1 ? kMarchTail : SPEC>(f, cx, cy, dir, t, t1, true);
         const int code = ray_code(f, t, t1, dir.x, dir.y, cx, cy);
         if (valid) (codes + sat)[lat] = code;
-        if (top) merge_top_quad(L, emis4, valid, code, sat + lat);
+        if (top) merge_top_quad(L, emis4, f.W, valid, code, sat + lat);
     }
 }
 

@@ -68,7 +68,7 @@ __device__ __forceinline__ void occ_bits_body(const float *__restrict__ depth, c
         for (int j = 0; j < 4; ++j)
             if (occ[j]) {
                 m |= 1u << j;
-                if (emis4) emis4[(size_t)(y0 + j) * W + x] = e[j];
+                if (emis4) emis4[emis_index(x, y0 + j, W)] = e[j];
             }
     }
     nib[w][lane] = (uint8_t)m;

@@ -190,7 +190,7 @@ __device__ inline int xcd_band(int b, int nb)
 struct LevelArgs {
     const uint8_t *sdf;      // distance codes, 16x8 tiles
     const float *emissive;   // [3][H][W]
-    const float4 *emis4;     // the same, interleaved (r, g, b, 0) per pixel, or nullptr (read the planes)
+    const float4 *emis4;     // the same, interleaved (r, g, b, 0) in 4x2-pixel blocks (emis_index), or nullptr (read the planes)
     const float2 *dirs;      // [N] unit directions of this level
     const void *upper;       // merged level i+1 (storage texels), nullptr at the top level
     void *out;               // merged level i (storage texels)

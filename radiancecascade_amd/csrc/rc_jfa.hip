@@ -88,7 +88,7 @@ __device__ __forceinline__ void seed_init_body(const float *__restrict__ depth, 
         if (y >= H) break;
         const size_t p = (size_t)y * W + x;
         seed[p] = occ[j] ? (((uint32_t)y << 16) | (uint32_t)x) : kFarSeed;
-        if (emis4 && occ[j]) emis4[p] = e[j];
+        if (emis4 && occ[j]) emis4[emis_index(x, y0 + j, W)] = e[j];
     }
 }
 

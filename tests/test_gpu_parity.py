@@ -508,6 +508,29 @@ def test_rays_leave_the_field_at_every_edge(rc, oracle, W, H, sdf):
                 assert np.array_equal(irr.cpu().numpy().view(np.uint32), irr32.view(np.uint32)), split
 
 
+@pytest.mark.parametrize("sdf", ["exact", "jfa"])
+@pytest.mark.parametrize("W,H", [(5, 3), (7, 9), (130, 67), (16384, 33), (16383, 18), (31, 16384)])
+def test_hits_take_their_own_pixels_emission(rc, oracle, W, H, sdf):
+    """Every emitter a colour of its own, so a hit that read another pixel of
+    the blocked emission shows: ragged blocks, the widest and tallest images."""
+    _say(f"emission blocks W={W} H={H} sdf={sdf}")
+    L = 3
+    rng = np.random.RandomState(W + H)
+    lit = rng.uniform(size=(H, W)) < 0.3
+    e = (rng.uniform(1.0, 2.0, (3, H, W)) * lit).astype(np.float32)
+    d = np.full((H, W), 0.5, np.float32)
+    ref = oracle.run(d, e, L, np.float32, sdf=sdf)  # by the same transform: the flood misses some nearest pixels
+    irr = torch.empty((3, H, W), dtype=torch.float32, device="cuda:0")
+    depth, emis = torch.from_numpy(d).cuda(), torch.from_numpy(e).cuda()
+    with rc.RadianceCascadeStage(W, H, levels=L) as st:
+        st.set_sdf_mode(sdf)
+        for split in (0, 1):
+            st.set_march(split, 1, 1)
+            st.run_device(depth, emis, irr)
+            torch.cuda.synchronize()
+            assert np.array_equal(irr.cpu().numpy().view(np.uint32), ref.view(np.uint32)), split
+
+
 @pytest.mark.parametrize("spec", [1, 2, 4])
 def test_persistent_march_is_bit_exact(rc, oracle, spec):
     """The persistent split march (split 2) stores the same ray codes and
