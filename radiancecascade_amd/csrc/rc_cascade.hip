@@ -692,42 +692,40 @@ __device__ inline void merge_top_quad(const MarchLevel &L, const float4 *__restr
     }
 }
 
-// A ray's march from t with SPEC samples per round: sample 0 at t and the
+// One round of a ray's march from t with SPEC samples: sample 0 at t and the
 // next ones where the ray goes if the step stays `guess` (every t is a whole
 // number below 2^24, so t + j guess is exact).  Sample j counts while the step
-// of every one before it was the guess; the last that counts gives the next t.
-// Branch-free, with the interval's end left to the loop: a sample beyond t1
-// can only leave t beyond t1.  Returns where t stopped: at the sample that
-// ended the ray (code 0: off-image or a hit), or at or past t1.
+// of every one before it was the guess; the last that counts gives the next t
+// and the next guess.  Branch-free, with the interval's end left to the caller:
+// a sample beyond t1 can only leave t beyond t1.  Returns whether the ray goes
+// on; otherwise t stopped at the sample that ended it (code 0: off-image or a
+// hit), or at or past t1.  all: every sample's step was the guess.
 template <int SPEC>
-__device__ __forceinline__ float march_speculative(const SdfField &f, float cx, float cy, float2 dir, float t,
-                                                   float t1, bool alive)
+__device__ __forceinline__ bool march_round(const SdfField &f, float cx, float cy, float2 dir, float t1, float &t,
+                                            float &guess, bool &all)
 {
-    float guess = 1.0f;
-    while (alive) {
-        float p[SPEC], step[SPEC];
-        uint32_t c[SPEC];
-        p[0] = t;
+    float p[SPEC], step[SPEC];
+    uint32_t c[SPEC];
+    p[0] = t;
 #pragma unroll
-        for (int j = 1; j < SPEC; ++j) p[j] = p[j - 1] + guess;
+    for (int j = 1; j < SPEC; ++j) p[j] = p[j - 1] + guess;
 #pragma unroll
-        for (int j = 0; j < SPEC; ++j)
-            c[j] = sdf_code(f, floor_i32(fmaf(p[j], dir.x, cx)), floor_i32(fmaf(p[j], dir.y, cy)));
+    for (int j = 0; j < SPEC; ++j)
+        c[j] = sdf_code(f, floor_i32(fmaf(p[j], dir.x, cx)), floor_i32(fmaf(p[j], dir.y, cy)));
 #pragma unroll
-        for (int j = 0; j < SPEC; ++j) step[j] = step_of_code(c[j]);
-        float at = p[0], by = step[0];
-        bool same = step[0] == guess;
+    for (int j = 0; j < SPEC; ++j) step[j] = step_of_code(c[j]);
+    float at = p[0], by = step[0];
+    bool same = step[0] == guess;
 #pragma unroll
-        for (int j = 1; j < SPEC; ++j) {
-            at = same ? p[j] : at;
-            by = same ? step[j] : by;
-            same = same && step[j] == guess;
-        }
-        t = at + by;
-        guess = by;
-        alive = by != 0.0f && t < t1;
+    for (int j = 1; j < SPEC; ++j) {
+        at = same ? p[j] : at;
+        by = same ? step[j] : by;
+        same = same && step[j] == guess;
     }
-    return t;
+    all = same;
+    t = at + by;
+    guess = by;
+    return by != 0.0f && t < t1;
 }
 
 // One ray per lane.  The median packet of 64 rays of a 1920x1080 frame ends
@@ -745,8 +743,21 @@ __device__ __forceinline__ float march_speculative(const SdfField &f, float cx, 
 //   longest, in 2,500 of the packets.  Frames of 1920x1080 took 129.1, 128.4,
 //   126.5 and 128.9 us with 8, 12, 16 and 24 plain samples, 151 with no others;
 //   6 and 8 samples a round 126.3 and 128.5.
-// Both with the field's zeros outside the image: march 60 -> 37 us at 1920x1080.
+// - That pays where rays run along a surface and repeat their step.  Among
+//   scattered pixels every step differs: a round takes one step for four
+//   loads, and the loads bound the launch (1920x1080 with a thousandth of the
+//   pixels lit: 587 us, 375 one sample a step).  So a wave first takes
+//   kTailProbe rounds, and guesses on to the end of its rays if 1 in
+//   kTailShare of them had all four steps alike; otherwise it takes kTailPlain
+//   samples one per step, probes again, and waits twice as long each time.
+//   That scene 373 us, lit boxes 122, 142 and 124 (121, 142 and 124 guessing
+//   always, 146 to 148 and 129 to 130 when the choice is made anew every round
+//   or few: it lies in the longest ray's chain).  What 8 packets a wave cost at
+//   3840x2160 stays: 2,960 us with a thousandth lit, 2,680 with 1, and boxes
+//   541 and 581.
+// Both kinds of scene with the field's zeros outside the image.
 constexpr int kMarchPlain = 16, kMarchTail = 4;
+constexpr int kTailProbe = 2, kTailShare = 16, kTailPlain = 32;
 //
 // What a packet needs beyond its rays is one wave-uniform tile (row, column,
 // slice) and lane constants: start points and addresses are a scalar part plus
@@ -814,14 +825,39 @@ __device__ __forceinline__ void march_packets(const SdfField &field, const March
         const float cy = (float)((int)__umul24((uint32_t)py, (uint32_t)spacing) + (spacing >> 1));
         float t = t0;
         bool alive = valid && t < t1;
+        float guess = 1.0f;
         if (SPEC == 1) {
             for (int step = 0; alive && step < kMarchPlain; ++step) {
                 const uint32_t c = sdf_code(f, floor_i32(fmaf(t, dir.x, cx)), floor_i32(fmaf(t, dir.y, cy)));
                 t = t + step_of_code(c);
                 alive = c != 0 && t < t1;
             }
+            int plain = kTailPlain;
+            while (const unsigned long long on = __ballot(alive)) {
+                int run = 0;
+                bool all;
+#pragma unroll 1
+                for (int round = 0; alive && round < kTailProbe; ++round) {
+                    alive = march_round<kMarchTail>(f, cx, cy, dir, t1, t, guess, all);
+                    run = all ? 1 : run;
+                }
+                if (__popcll(__ballot(run != 0)) * kTailShare >= __popcll(on)) {
+                    while (alive) alive = march_round<kMarchTail>(f, cx, cy, dir, t1, t, guess, all);
+                    break;
+                }
+#pragma unroll 1
+                for (int step = 0; alive && step < plain; ++step) {
+                    const uint32_t c = sdf_code(f, floor_i32(fmaf(t, dir.x, cx)), floor_i32(fmaf(t, dir.y, cy)));
+                    guess = step_of_code(c);
+                    t = t + guess;
+                    alive = c != 0 && t < t1;
+                }
+                plain *= 2;  // a ray takes fewer than 2^16 samples (t1 < 2^16, steps of 1 at least)
+            }
+        } else {
+            bool all;
+            while (alive) alive = march_round<SPEC>(f, cx, cy, dir, t1, t, guess, all);
         }
-        if (alive) t = march_speculative<SPEC == 1 ? kMarchTail : SPEC>(f, cx, cy, dir, t, t1, true);
         const int code = ray_code(f, t, t1, dir.x, dir.y, cx, cy);
         if (valid) (codes + sat)[lat] = code;
         if (top) merge_top_quad(L, emis4, f.W, valid, code, sat + lat);
