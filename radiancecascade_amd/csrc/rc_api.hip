@@ -355,7 +355,10 @@ static MarchAllArgs march_all_args(const rc_ctx *c, bool gated = false)
         l.dir_off = (int)c->dir_off[i];
         m.total_rays += (uint32_t)((int64_t)l.PX * l.PY * l.N);
     }
-    for (int j = 0; j < m.nlev; ++j) march_level_blocks(m.lev[j], spec, rays, slots);
+    for (int j = 0; j < m.nlev; ++j) {
+        march_level_blocks(m.lev[j], spec, rays, slots);
+        if (gated) m.lev[j].blocks = std::min(m.lev[j].blocks, std::max(1, kGatedWaves / m.nlev));
+    }
     m.codes_base = c->codes;
     m.dirs_base = c->dirs;
     m.emis4 = c->emis4;

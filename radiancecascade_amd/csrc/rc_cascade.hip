@@ -770,7 +770,7 @@ template <int SPEC, bool GATED>
 __device__ __forceinline__ void march_packets(const SdfField &field, const MarchLevel &L, int lb,
                                               const float4 *__restrict__ emis4)
 {
-    const int lane = (int)threadIdx.x;
+    const int lane = (int)threadIdx.x & 63;
     SdfField f = field;
     f.W = uniform(f.W);
     f.H = uniform(f.H);
@@ -913,12 +913,22 @@ __global__ __launch_bounds__(kMarchBlock) void k_march_all(MarchAllArgs a)
 }
 
 // The tile fallback's split march: nothing when no tile is flagged, and only
-// the probes the flagged tiles need.
-__global__ __launch_bounds__(kMarchBlock) void k_march_gated(MarchAllArgs a)
+// the probes the flagged tiles need.  A frame with no flagged tile pays for
+// handing the workgroups out, so there are few: two waves each, and at most
+// kGatedWaves waves a launch, which then take more packets.  Unused, with one
+// wave each and no limit, it took 60.2, 82.0, 110.3 and 283 us of frames of
+// 700x400, 1366x768, 1920x1080 and 3840x2160, 57.5, 77.0, 98.0 and 265 so
+// (56.4, 77.1, 99.9 and 288 when the fallback marched in place).  With about
+// 40 % of the tiles flagged 94.4, 136.3, 180.2 and 596 us, 94.1, 137.9, 182.0
+// and 592 so; with all of them 97.2, 145.4, 203 and 782, 97.0, 146.9, 213.5
+// and 785 (four waves and no limit: 97.4, 147.1, 213.5 and 807; 16,384 waves
+// of one: 98.9, 147.5, 211 and 806).
+__global__ __launch_bounds__(kGatedBlock) void k_march_gated(MarchAllArgs a)
 {
     const MarchLevel &L = a.lev[blockIdx.y];
-    if ((int)blockIdx.x >= L.blocks || *a.gate == 0) return;
-    march_packets<1, true>(sdf_field(a.sdf, a.W, a.H), L, (int)blockIdx.x, a.emis4);
+    const int wave = (int)blockIdx.x * (kGatedBlock / 64) + uniform((int)threadIdx.x >> 6);
+    if (wave >= L.blocks || *a.gate == 0) return;
+    march_packets<1, true>(sdf_field(a.sdf, a.W, a.H), L, wave, a.emis4);
 }
 
 // The split march over a work list of (view, level) jobs, blocks in launch
@@ -1177,7 +1187,8 @@ hipError_t launch_march_all(const MarchAllArgs &a, int spec, int m, hipStream_t 
     for (int i = 0; i < a.nlev; ++i) blocks = a.lev[i].blocks > blocks ? a.lev[i].blocks : blocks;
     if (blocks <= 0) return hipSuccess;
     if (a.gate) {
-        hipLaunchKernelGGL(k_march_gated, dim3(blocks, a.nlev), dim3(kMarchBlock), 0, s, a);
+        constexpr int waves = kGatedBlock / 64;
+        hipLaunchKernelGGL(k_march_gated, dim3((blocks + waves - 1) / waves, a.nlev), dim3(kGatedBlock), 0, s, a);
         return hipGetLastError();
     }
     switch (spec) {

@@ -204,6 +204,8 @@ struct LevelArgs {
     const uint8_t *need;     // gated merge: [PY][PX] probes to compute; the others are left untouched
 };
 
+// the gated march: threads of a workgroup, and waves of a launch at most
+constexpr int kGatedBlock = 128, kGatedWaves = 32768;
 // k_march_all: every level >= 1 in one launch (level-major, top level first).
 struct MarchLevel {
     const float2 *dirs;

@@ -78,3 +78,56 @@ def test_scattered_pixels_are_no_slower_than_one_sample_a_step(rc):
             st.set_march(split, 1, 1)
             us[split] = _us(lambda: st.run_device(d, e, irr))
     assert us[1] <= us[0], us
+
+
+def _boxes(rc, W, H, seed):
+    d, a, e = (torch.empty(s, device="cuda:0") for s in ((H, W), (3, H, W), (3, H, W)))
+    rc.gbuffer_raster(rc.scene_generate(seed, 32, 4), W, H, d, a, e)
+    return d, e
+
+
+@pytest.mark.parametrize("W,H,L", [(1366, 768, 6), (1921, 1079, 3)])
+def test_fallback_march_of_several_packets_a_wave(rc, W, H, L):
+    """A fallback launch of more packets than its waves may be: flagged tiles
+    equal the plain level 1 bit for bit, the others the learned one, with
+    another scene's codes left in the buffer."""
+    irr = torch.empty((3, H, W), device="cuda:0")
+    with rc.RadianceCascadeStage(W, H, levels=L) as plain, rc.RadianceCascadeStage(W, H, levels=L) as st:
+        st.load_weights()
+        py, px = plain.level_shape(1)[:2]
+        a1 = {k: torch.empty(plain.level_shape(1), device="cuda:0") for k in "plf"}
+        terr = torch.empty(st.surrogate_shapes()["tiles"], device="cuda:0")
+        for seed in (2, 3):
+            d, e = _boxes(rc, W, H, seed)
+            plain.run_device(d, e, irr)
+            plain.debug_level(1, a1["p"])
+            st.set_surrogate(True)
+            st.run_device(d, e, irr)
+            st.debug_level(1, a1["l"])
+            st.debug_surrogate(tile_err=terr)
+            thr = float(terr.median())
+            st.set_surrogate(True, threshold=thr)
+            st.run_device(d, e, irr)
+            st.debug_level(1, a1["f"])
+            torch.cuda.synchronize()
+            flag = np.repeat(np.repeat(~(terr.cpu().numpy() <= thr), 16, axis=0), 16, axis=1)[:py, :px]
+            assert 0 < flag.sum() < flag.size
+            f, p, l = (a1[k].cpu().numpy().view(np.uint32) for k in "fpl")
+            assert np.array_equal(f[flag], p[flag]) and np.array_equal(f[~flag], l[~flag]), seed
+
+
+def test_an_unused_fallback_costs_its_launches(rc):
+    """A learned frame with the fallback on and no tile flagged: 1.31 times the
+    frame without it where the fallback marched level by level, 1.30 now, 1.47
+    when its march handed out a workgroup per wave of the whole frame."""
+    W, H = 1920, 1080
+    d, e = _boxes(rc, W, H, 3)
+    irr = torch.empty((3, H, W), device="cuda:0")
+    us = {}
+    with rc.RadianceCascadeStage(W, H) as st:
+        st.load_weights()
+        for thr in (float("inf"), 1e30):
+            st.set_surrogate(True, threshold=thr)
+            us[thr] = _us(lambda: st.run_device(d, e, irr))
+        assert st.stats().flagged_tiles == 0
+    assert us[1e30] <= 1.4 * us[float("inf")], us
