@@ -354,7 +354,10 @@ rc_status rc_surrogate_load(rc_ctx *ctx, const void *buf, uint64_t size);
  * out: [n][64] raw outputs z.  rc_mlp_gradient: targets [n][48] normalised
  * residuals; grad: RC_MLP_PARAMS fp32 of the batch-mean loss
  * L = sum (z - t)^2 / (48 n) + 0.05 sum (z_48 - log(mse_s + 1e-2))^2 / n;
- * loss: 1 float.  rc_mlp_adam: one Adam step (0.9, 0.999, 1e-8) with grad. */
+ * loss: 1 float; with a stream of the caller's it returns when they are
+ * written, on the null stream (and on one that is being captured) it is stream
+ * ordered like rc_mlp_forward and rc_mlp_adam.  rc_mlp_adam: one Adam step
+ * (0.9, 0.999, 1e-8) with grad. */
 rc_status rc_mlp_forward(rc_ctx *ctx, const float *feats_dev, uint32_t n, float *out_dev, void *stream);
 rc_status rc_mlp_gradient(rc_ctx *ctx, const float *feats_dev, const float *targets_dev, uint32_t n, float *grad_dev,
                           float *loss_dev, void *stream);
