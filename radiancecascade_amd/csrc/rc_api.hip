@@ -898,8 +898,11 @@ static rc_status ensure_mlp_scratch(rc_ctx *c, int parts, int rows)
     return RC_OK;
 }
 
+// Called without a stream: work of the context on any stream may still read
+// the network it replaces.
 static rc_status mlp_upload(rc_ctx *c, const float *params, const float *mean, const float *istd, float out_scale)
 {
+    HIP_TRY(c, hipDeviceSynchronize());
     HIP_TRY(c, hipMemcpy(c->mlp.master, params, kMlpParams * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(c, hipMemcpy(c->mlp.in_mean, mean, kMlpIn * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(c, hipMemcpy(c->mlp.in_istd, istd, kMlpIn * sizeof(float), hipMemcpyHostToDevice));

@@ -97,3 +97,48 @@ def test_gradient_in_a_captured_graph(rc):
             torch.cuda.synchronize()
             st.mlp_gradient(x, t, ge, le)
             assert torch.equal(g, ge) and torch.equal(lo, le), k
+
+
+@pytest.mark.parametrize("call", ["forward", "gradient", "frame"])
+def test_a_new_network_waits_for_the_old_ones_work(rc, call):
+    """Work queued on another stream before mlp_set uses the network it was
+    given."""
+    n = 20000
+    rng = np.random.default_rng(6)
+    x = torch.from_numpy(rng.standard_normal((n, 64)).astype(np.float32)).cuda()
+    t = torch.from_numpy(rng.standard_normal((n, 48)).astype(np.float32)).cuda()
+    W, H = 320, 200
+    e = torch.from_numpy((rng.uniform(size=(3, H, W)) < 0.01).astype(np.float32)).cuda()
+    d = torch.full((H, W), 0.5, device="cuda:0")
+    with rc.RadianceCascadeStage(W, H, levels=4) as st:
+        st.set_surrogate(True)
+
+        def go(stream):
+            if call == "forward":
+                out = torch.zeros((n, 64), device="cuda:0")
+                torch.cuda.synchronize()
+                return lambda: st.mlp_forward(x, out, stream=stream), [out]
+            if call == "gradient":
+                out = [torch.zeros(rc._abi.MLP_PARAMS, device="cuda:0"), torch.zeros(1, device="cuda:0")]
+                torch.cuda.synchronize()
+                return lambda: st.mlp_gradient(x, t, *out, stream=stream), out
+            out = torch.zeros_like(e)
+            torch.cuda.synchronize()
+            return lambda: st.run_device(d, e, out, stream=stream), [out]
+
+        side = torch.cuda.Stream()
+        st.mlp_set(*_net(rc, 7))
+        run, want = go(side)
+        run()
+        torch.cuda.synchronize()
+        run, got = go(side)
+        keep = _busy(side)
+        run()
+        st.mlp_set(*_net(rc, 8))
+        torch.cuda.synchronize()
+        del keep
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        run, other = go(side)
+        run()
+        torch.cuda.synchronize()
+        assert not torch.equal(other[0], want[0])
