@@ -158,10 +158,12 @@ rc_status rc_run_device(rc_ctx *ctx, const rc_gbuffer *dev, float *irradiance_de
  * harnesses that forbid hipMalloc).  The plain GI frame of rc_run_device --
  * linear depth, fp32 storage; the irradiance is equal bit for bit -- with no
  * context: its working buffers (jump-flood fields, distance field, merged
- * levels) live in a static 64 MiB device array that each GPU holds until the
- * process ends (enough for 1920x1080 with 6 levels; rc_noalloc_scratch_bytes
- * gives a size's need, larger sizes are refused with RC_ERR_INVALID), and
- * its direction tables in a static array set on the first call on a device.
+ * levels) live in a static device array that each GPU holds until the process
+ * ends (64 MiB, enough for 1920x1080 with 6 levels, and 8 rows of the distance
+ * field more, which a height that is a multiple of 8 needs;
+ * rc_noalloc_scratch_bytes gives a size's need, larger sizes are refused with
+ * RC_ERR_INVALID), and its direction tables in a static array set on the first
+ * call on a device.
  * It calls no hipMalloc, hipFree or other allocating routine.  Runs on the
  * current device, stream ordered.  Every call on one GPU shares that GPU's
  * scratch: calls that overlap on one GPU (several streams or threads) race.

@@ -36,8 +36,9 @@ constexpr size_t kNoAllocScratchBytes = 64ull << 20;
 constexpr int kNoAllocMaxLevels = 7;
 constexpr int kNoAllocDirs = 4 * ((1 << (2 * kNoAllocMaxLevels)) - 1) / 3;  // sum of N_i, i < 7
 
-// The distance field, last in the layout, has rows beyond the image's; those
-// that make it a band of 8 rows more lie past the bytes counted.
+// Where the height is a multiple of 8 the distance field's row of zeros below
+// the image takes a band of 8 rows of its own; sizes are taken or refused
+// without it, so the array has the widest one on top.
 constexpr size_t kNoAllocFieldPad = 8 * RC_MAX_DIM;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes + kNoAllocFieldPad];
 static __device__ __align__(256) float2 scratch_dirs[kNoAllocDirs];
@@ -53,6 +54,7 @@ static std::mutex g_noalloc_mu;
 
 struct NoAllocLayout {
     size_t bits, ends, sdf, level[RC_MAX_LEVELS], total;
+    bool fits;
 };
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -65,12 +67,16 @@ static NoAllocLayout noalloc_layout(int W, int H, int L)
     off = align256(off + edt_bits_bytes(W, H));
     m.ends = off;
     off = align256(off + edt_ends_bytes(W, H));
+    m.sdf = off;
+    off = align256(off + sdf_elems(W, H));
     for (int i = 1; i < L; ++i) {
         m.level[i] = off;
         off = align256(off + (size_t)grid_dim(W, i) * grid_dim(H, i) * (num_dirs(i) / 4) * sizeof(float4));
     }
-    m.sdf = off;
-    m.total = align256(off + (size_t)sdf_width(W) * ((H + 7) & ~7));
+    m.total = off;
+    static_assert(RC_MAX_DIM % 32 == 0, "the widest band is whole 256-byte steps: none is larger");
+    const size_t band = align256(sdf_elems(W, H)) - align256((size_t)sdf_width(W) * ((H + 7) & ~7));
+    m.fits = off <= kNoAllocScratchBytes + band;
     return m;
 }
 
@@ -141,7 +147,7 @@ rc_status rc_run_device_noalloc(uint32_t width, uint32_t height, uint32_t levels
         return nfail(RC_ERR_INVALID, "rc_run_device_noalloc: levels must be 1.." + std::to_string(kNoAllocMaxLevels));
     const int W = (int)width, H = (int)height, L = (int)levels;
     const NoAllocLayout lay = noalloc_layout(W, H, L);
-    if (lay.total > kNoAllocScratchBytes)
+    if (!lay.fits)
         return nfail(RC_ERR_INVALID, "rc_run_device_noalloc: " + std::to_string(W) + "x" + std::to_string(H) + " with " +
                                          std::to_string(L) + " levels needs " + std::to_string(lay.total) +
                                          " bytes of scratch; the static scratch holds " +
