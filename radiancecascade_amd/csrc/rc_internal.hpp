@@ -10,8 +10,12 @@ namespace rc {
 
 // ---- scene (rc_scene.hip) ---------------------------------------------------
 void scene_generate(uint64_t seed, int n_boxes, int n_emissive, rc_box *boxes);
-// up to kRasterArgBoxes boxes given by the host, passed as kernel arguments
-constexpr int kRasterArgBoxes = 32;
+// up to kRasterArgBoxes boxes given by the host, passed as kernel arguments: as
+// many as fit the 4 KB of a launch beside the other 40 bytes.  With a list in
+// device memory (an allocation, a copy and a free around the kernel) 33 and 42
+// boxes took 43 to 44 us at 64x64 and 66 and 72 at 1920x1080, 28 to 30 and 54
+// and 58 so.
+constexpr int kRasterArgBoxes = 42;
 hipError_t launch_raster_args(const rc_box *boxes, int n, int W, int H, float *depth, float *albedo, float *emissive,
                               hipStream_t stream);
 hipError_t launch_raster(const double *boxes_dev, int n, int W, int H, float *depth, float *albedo, float *emissive,

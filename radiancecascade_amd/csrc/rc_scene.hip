@@ -70,6 +70,7 @@ constexpr int kRasterRows = 16, kRasterChunk = 32;
 struct RasterArgs {
     double box[kRasterArgBoxes * 12];
 };
+static_assert(sizeof(RasterArgs) + 40 <= 4096 && sizeof(RasterArgs) + 40 + 12 * sizeof(double) > 4096, "what a launch holds");
 
 struct Slab {
     double n, f;  // nearer and farther plane
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(kBlock) void k_raster(const double *__restrict__ bo
     raster_body(boxes, n, W, H, depth, albedo, emissive);
 }
 
-// A box list short enough to travel with the launch (3 KB of kernel
+// A box list short enough to travel with the launch (4 KB of kernel
 // arguments): no device allocation and no copy before the kernel.
 __global__ __launch_bounds__(kBlock) void k_raster_args(RasterArgs r, int n, int W, int H, float *__restrict__ depth,
                                                         float *__restrict__ albedo, float *__restrict__ emissive)
