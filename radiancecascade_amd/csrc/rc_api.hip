@@ -1185,7 +1185,7 @@ rc_status rc_debug_march(rc_ctx *c, uint32_t level, int32_t *hit_dev, int64_t *i
         if (level == 0) return fail(c, RC_ERR_INVALID, "rc_debug_march: level 0 has no split-march decode");
         const MarchAllArgs m = march_all_args(c);
         HIP_TRY(c, hipMemsetAsync(index_dev, 0xFF, rays * sizeof(int64_t), s));  // -1: no slot
-        HIP_TRY(c, launch_ray_decode(m.lev[c->L - 1 - (int)level], index_dev, s));
+        HIP_TRY(c, launch_ray_decode(m.lev[c->L - 1 - (int)level], c->march_m, index_dev, s));
     }
     return RC_OK;
 }

@@ -621,34 +621,81 @@ __device__ inline void decode_ray(const MarchLevel &L, int ray, int &px, int &py
     else if (px >= L.PX) { ++py; px -= L.PX; }
 }
 
-// Split-march slot -> (px, py, k).  Wave tiles: slot = T*64 + lane, T = (tile
-// row * ntx + tile column) * slices + slice, lane = (probe in the tile,
-// direction in the slice) with the direction fastest; false for the lanes of a
-// ragged edge tile that fall outside the probe grid.  Rays with nearby start
-// points and directions share a wave, so their march lengths are alike.
-// Canonical order is the wave tile of one probe x 64 directions, or, for
-// level 1's 16 directions (kd_log = 0), the canonical index itself.  T is
-// wave-uniform, so the tile's row and column are scalar arithmetic: the
-// quotient's estimate by the reciprocal is off by at most one either way.
-__device__ inline bool decode_slot(const MarchLevel &L, int T, int lane, int &px, int &py, int &k)
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// The order of a level's rays over the split march's slots.  Wave tiles: slot =
+// T*64 + lane, T = (tile row * ntx + tile column) * slices + slice, lane =
+// (probe in the tile, direction in the slice) with the direction fastest.  Rays
+// with nearby start points and directions share a wave, so their march lengths
+// are alike.  Canonical order is the wave tile of one probe x 64 directions,
+// or, for level 1's 16 directions (wrap), the canonical index itself: 4
+// consecutive probes, which may wrap to the next row.
+// A packet T is one wave-uniform tile (row, column, slice) and lane constants:
+// start points and addresses are a part of T's plus a lane's, and the level's
+// fields stay in scalar registers (read from the arguments per packet, one
+// after another, they took a launch without march and stores to 14.7 us at
+// 1920x1080).  Every march of the split launch and the readback of its order
+// place rays by this.
+struct RayOrder {
+    int PX, PY, log2n, slots, tx_log, ty_log, ntx, rcp, kd_log, ns_log, smask;
+    bool wrap;
+    int lane, lk, lx, ly;
+    uint32_t lat;  // the lane's part of its rays' canonical index
+};
+__device__ __forceinline__ RayOrder ray_order(const MarchLevel &L, int lane)
 {
-    if (L.map == 0 && L.kd_log == 0) {
-        const int ray = T * 64 + lane;
-        const bool in = ray < (int)L.slots;
+    RayOrder o;
+    o.PX = uniform(L.PX), o.PY = uniform(L.PY), o.log2n = uniform(L.log2n), o.slots = uniform((int)L.slots);
+    o.tx_log = uniform(L.tx_log), o.ty_log = uniform(L.ty_log);
+    o.ntx = uniform(L.ntx), o.rcp = uniform((int)L.rcp_ntx);
+    o.wrap = L.map == 0 && L.kd_log == 0;
+    o.kd_log = uniform(o.wrap ? 4 : L.kd_log), o.ns_log = o.log2n - o.kd_log;
+    o.smask = (1 << o.ns_log) - 1;
+    o.lane = lane;
+    o.lk = lane & ((1 << o.kd_log) - 1);
+    const int pl = lane >> o.kd_log;
+    o.lx = pl & ((1 << o.tx_log) - 1), o.ly = pl >> o.tx_log;
+    o.lat = o.wrap ? (uint32_t)lane
+                   : ((__umul24((uint32_t)o.ly, (uint32_t)o.PX) + (uint32_t)o.lx) << o.log2n) + (uint32_t)o.lk;
+    return o;
+}
+// The lane's direction in packet T, as an offset into the level's table: the
+// part of T's (lk is the lane's).
+__device__ __forceinline__ int ray_slice(const RayOrder &o, int T) { return o.wrap ? 0 : (T & o.smask) << o.kd_log; }
+// The probe of the lane's ray in packet T, and at: the part of T's of its
+// canonical index (the other is lat).  False for a lane without a ray: past the
+// last slot, or outside the probe grid in a ragged edge tile.  The quotient's
+// estimate by the reciprocal is off by at most one either way.
+__device__ __forceinline__ bool ray_place(const RayOrder &o, const MarchLevel &L, int T, int &px, int &py, uint32_t &at)
+{
+    if (o.wrap) {
+        int k;
+        const int ray = T * 64 + o.lane;
+        const bool in = ray < o.slots;
         decode_ray(L, in ? ray : 0, px, py, k);
+        at = (uint32_t)T * 64;
         return in;
     }
-    const int ns_log = L.log2n - L.kd_log;
-    const uint32_t tt = (uint32_t)T >> ns_log, ntx = (uint32_t)L.ntx;
-    uint32_t ty = __umulhi(tt, L.rcp_ntx);
+    const uint32_t tt = (uint32_t)T >> o.ns_log, ntx = (uint32_t)o.ntx;
+    uint32_t ty = __umulhi(tt, (uint32_t)o.rcp);
     if (ty * ntx > tt) --ty;
     if (tt - ty * ntx >= ntx) ++ty;
-    const uint32_t tx = tt - ty * ntx;
-    const int pl = lane >> L.kd_log;
-    k = ((T & ((1 << ns_log) - 1)) << L.kd_log) | (lane & ((1 << L.kd_log) - 1));
-    px = (int)(tx << L.tx_log) | (pl & ((1 << L.tx_log) - 1));
-    py = (int)(ty << L.ty_log) | (pl >> L.tx_log);
-    return px < L.PX && py < L.PY;
+    const int sx = (int)(tt - ty * ntx) << o.tx_log, sy = (int)ty << o.ty_log;
+    px = sx + o.lx;
+    py = sy + o.ly;
+    at = ((uint32_t)(sy * o.PX + sx) << o.log2n) + (uint32_t)ray_slice(o, T);
+    return px < o.PX && py < o.PY;
+}
+// The packets of wave `wave`: first, first + step, ... below end.  One ray a
+// lane at a time: a grid's width of waves apart; M: the M next to each other.
+struct Packets {
+    int first, step, end;
+};
+__device__ __forceinline__ Packets wave_packets(const MarchLevel &L, int wave, int m)
+{
+    const int all = uniform((int)((L.slots + 63) >> 6));
+    if (m == 1) return Packets{wave, uniform(L.blocks), all};
+    return Packets{wave * m, 1, min(wave * m + m, all)};
 }
 
 // All levels >= 1 marched by one launch; each ray's code (hit pixel, -1 left
@@ -758,13 +805,6 @@ __device__ __forceinline__ bool march_round(const SdfField &f, float cx, float c
 // Both kinds of scene with the field's zeros outside the image.
 constexpr int kMarchPlain = 16, kMarchTail = 4;
 constexpr int kTailProbe = 2, kTailShare = 16, kTailPlain = 32;
-//
-// What a packet needs beyond its rays is one wave-uniform tile (row, column,
-// slice) and lane constants: start points and addresses are a scalar part plus
-// a lane part, and the level's fields stay in scalar registers (read from the
-// arguments per packet, one after another, they took a launch without march
-// and stores to 14.7 us at 1920x1080).
-__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 template <int SPEC, bool GATED>
 __device__ __forceinline__ void march_packets(const SdfField &field, const MarchLevel &L, int lb,
@@ -775,49 +815,24 @@ __device__ __forceinline__ void march_packets(const SdfField &field, const March
     f.W = uniform(f.W);
     f.H = uniform(f.H);
     f.skip = uniform(f.skip);
-    const int PX = uniform(L.PX), PY = uniform(L.PY), log2n = uniform(L.log2n), nw = uniform(L.blocks);
-    const int end = uniform((int)((L.slots + 63) >> 6)), slots = uniform((int)L.slots);
-    const int tx_log = uniform(L.tx_log), ty_log = uniform(L.ty_log);
-    const int spacing = uniform((int)L.spacing), ntx = uniform(L.ntx), rcp = uniform((int)L.rcp_ntx);
+    const RayOrder o = ray_order(L, lane);
+    const int spacing = uniform((int)L.spacing);
     const float t0 = __int_as_float(uniform(__float_as_int(L.t0))), t1 = __int_as_float(uniform(__float_as_int(L.t1)));
     const float2 *dirs = L.dirs;
     int *codes = L.codes;
     const bool top = L.merged != nullptr;
-    // level 1 in canonical order: 4 consecutive probes x 16 directions, which may wrap to the next row
-    const bool wrap = L.map == 0 && L.kd_log == 0;
-    const int kd_log = uniform(wrap ? 4 : L.kd_log), ns_log = log2n - kd_log;
-    const int smask = (1 << ns_log) - 1;
-    const int lk = lane & ((1 << kd_log) - 1), pl = lane >> kd_log;
-    const int lx = pl & ((1 << tx_log) - 1), ly = pl >> tx_log;
-    const uint32_t lat = wrap ? (uint32_t)lane : ((__umul24((uint32_t)ly, (uint32_t)PX) + (uint32_t)lx) << log2n) + (uint32_t)lk;
-    auto direction = [&](int T) -> float2 { return (dirs + (wrap ? 0 : (T & smask) << kd_log))[lk]; };
+    auto direction = [&](int T) -> float2 { return (dirs + ray_slice(o, T))[o.lk]; };
 
-    float2 next = direction(lb);
-    for (int T = lb; T < end; T += nw) {
+    const Packets p = wave_packets(L, lb, 1);
+    float2 next = direction(p.first);
+    for (int T = p.first; T < p.end; T += p.step) {
         const float2 dir = next;
-        next = direction(T + nw);
+        next = direction(T + p.step);
         int px, py;
-        bool valid;
-        uint32_t sat;  // the scalar part of the rays' canonical index
-        if (wrap) {
-            int k;
-            const int ray = T * 64 + lane;
-            valid = ray < slots;
-            decode_ray(L, valid ? ray : 0, px, py, k);
-            sat = (uint32_t)T * 64;
-        } else {
-            const uint32_t tt = (uint32_t)T >> ns_log;
-            uint32_t ty = __umulhi(tt, (uint32_t)rcp);
-            if (ty * (uint32_t)ntx > tt) --ty;
-            if (tt - ty * (uint32_t)ntx >= (uint32_t)ntx) ++ty;
-            const int sx = (int)(tt - ty * (uint32_t)ntx) << tx_log, sy = (int)ty << ty_log;
-            px = sx + lx;
-            py = sy + ly;
-            valid = px < PX && py < PY;
-            sat = ((uint32_t)(sy * PX + sx) << log2n) + (uint32_t)((T & smask) << kd_log);
-        }
+        uint32_t at;
+        bool valid = ray_place(o, L, T, px, py, at);
         if (GATED) {
-            valid = valid && L.need[py * PX + px] != 0;
+            valid = valid && L.need[py * o.PX + px] != 0;
             if (!__any(valid)) continue;
         }
         // (p + 1/2) spacing, a whole number: spacing is even
@@ -859,8 +874,8 @@ __device__ __forceinline__ void march_packets(const SdfField &field, const March
             while (alive) alive = march_round<SPEC>(f, cx, cy, dir, t1, t, guess, all);
         }
         const int code = ray_code(f, t, t1, dir.x, dir.y, cx, cy);
-        if (valid) (codes + sat)[lat] = code;
-        if (top) merge_top_quad(L, emis4, f.W, valid, code, sat + lat);
+        if (valid) (codes + at)[o.lat] = code;
+        if (top) merge_top_quad(L, emis4, f.W, valid, code, at + o.lat);
     }
 }
 
@@ -873,19 +888,18 @@ __device__ __forceinline__ void march_all_body(const uint8_t *sdf_codes, int W, 
         march_packets<SPEC, false>(f, L, lb, emis4);
         return;
     }
-    const int base = lb * kMarchBlock * M + (int)threadIdx.x;
-    const int total = (int)L.slots;
+    const RayOrder o = ray_order(L, (int)threadIdx.x);
+    const Packets p = wave_packets(L, lb, M);
 
-    int j = 0, ray = base;
+    int j = 0, T = p.first;
     bool valid = false;      // the slot holds a ray of the grid
     uint32_t at = 0;         // its canonical index (where its code goes)
     Ray r;
     auto start = [&]() {
-        const int slot = ray < total ? ray : 0;
-        int px, py, k;
-        valid = decode_slot(L, slot >> 6, slot & 63, px, py, k) && ray < total;
-        at = ((__umul24((uint32_t)py, (uint32_t)L.PX) + (uint32_t)px) << L.log2n) + (uint32_t)k;
-        const float2 dir = L.dirs[k];
+        int px, py;
+        valid = ray_place(o, L, T < p.end ? T : 0, px, py, at) && T < p.end;
+        at += o.lat;
+        const float2 dir = L.dirs[at & (uint32_t)(L.N - 1)];
         r = ray_begin(((float)px + 0.5f) * L.spacing, ((float)py + 0.5f) * L.spacing, dir.x, dir.y, L.t0, L.t1,
                       valid);
     };
@@ -894,7 +908,7 @@ __device__ __forceinline__ void march_all_body(const uint8_t *sdf_codes, int W, 
         if (r.alive) ray_round<SPEC>(r, f, L.t1);
         if (j < M && !r.alive) {
             if (valid) L.codes[at] = r.code;
-            ray += kMarchBlock;
+            T += p.step;
             if (++j < M) start();
         }
         if (!__any(j < M)) break;
@@ -1045,17 +1059,18 @@ __global__ __launch_bounds__(kBlock) void k_march_persist(MarchAllArgs a)
     }
 }
 
-// The split march's decode of every slot of one level, recomposed into the
-// canonical index it stands for (parity readback: equal to the slot number
-// when the decode is right).
-// For every slot of a level's split march, its ray's canonical index gets
-// the slot number (the slot that marches it).
-__global__ __launch_bounds__(kBlock) void k_ray_decode(MarchLevel l, int64_t *__restrict__ index)
+// For every slot of a level's split march, its ray's canonical index gets the
+// slot number: the packets of the march's own waves, placed as it places them
+// (parity readback).
+__global__ __launch_bounds__(kMarchBlock) void k_ray_decode(MarchLevel l, int m, int64_t *__restrict__ index)
 {
-    const int slot = (int)(blockIdx.x * kBlock + threadIdx.x);
-    if (slot >= (int)l.slots) return;
-    int px, py, k;
-    if (decode_slot(l, slot >> 6, slot & 63, px, py, k)) index[((int64_t)py * l.PX + px) * l.N + k] = slot;
+    const RayOrder o = ray_order(l, (int)threadIdx.x);
+    const Packets p = wave_packets(l, (int)blockIdx.x, m);
+    for (int T = p.first; T < p.end; T += p.step) {
+        int px, py;
+        uint32_t at;
+        if (ray_place(o, l, T, px, py, at)) index[at + o.lat] = (int64_t)T * 64 + o.lane;
+    }
 }
 
 template <Storage S>
@@ -1343,12 +1358,10 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
     l.blocks = (int)(((int64_t)l.slots + per - 1) / per);
 }
 
-hipError_t launch_ray_decode(const MarchLevel &l, int64_t *index, hipStream_t s)
+hipError_t launch_ray_decode(const MarchLevel &l, int rays_per_lane, int64_t *index, hipStream_t s)
 {
-    const int64_t total = (int64_t)l.slots;
-    const unsigned blocks = (unsigned)((total + kBlock - 1) / kBlock);
-    if (blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_ray_decode, dim3(blocks), dim3(kBlock), 0, s, l, index);
+    if (l.blocks <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_ray_decode, dim3(l.blocks), dim3(kMarchBlock), 0, s, l, rays_per_lane, index);
     return hipGetLastError();
 }
 

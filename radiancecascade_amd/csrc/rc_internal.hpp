@@ -301,7 +301,7 @@ hipError_t launch_level0_gather(const LevelArgs &a, Storage st, float *irradianc
                                 hipStream_t s);
 hipError_t launch_level_to_f32(const void *level, Storage st, size_t texels, float *out, hipStream_t s);
 // canonical ray index of each slot as the split march decodes it (parity readback)
-hipError_t launch_ray_decode(const MarchLevel &l, int64_t *index, hipStream_t s);
+hipError_t launch_ray_decode(const MarchLevel &l, int rays_per_lane, int64_t *index, hipStream_t s);
 
 // ---- error norms (rc_norms.hip) ---------------------------------------------
 size_t norm_workspace_bytes();

@@ -131,3 +131,41 @@ def test_an_unused_fallback_costs_its_launches(rc):
             us[thr] = _us(lambda: st.run_device(d, e, irr))
         assert st.stats().flagged_tiles == 0
     assert us[1e30] <= 1.4 * us[float("inf")], us
+
+
+@pytest.mark.parametrize("march", [(1, 1, 1), (1, 2, 1), (1, 4, 1), (1, 1, 2), (1, 2, 4), (1, 1, 8), (2, 1, 1)])
+@pytest.mark.parametrize("W,H,L", [(413, 211, 6), (97, 61, 4), (1030, 17, 3), (1366, 768, 6)])
+def test_every_form_and_order_marches_every_ray(rc, oracle, march, W, H, L):
+    """Each form of the split march in each order of its lanes, after another
+    form left the codes and levels of a frame in which every ray hits: codes
+    and irradiance are the oracle's, and the march's own packets place every
+    ray in one slot.  The larger size takes two packets a wave."""
+    e_lit = torch.ones((3, H, W), device="cuda:0")
+    d, e = _boxes(rc, W, H, 4)
+    dn, en = d.cpu().numpy(), e.cpu().numpy()
+    want = oracle.run(dn, en, L, np.float32)
+    field = oracle.sdf_from_d2(oracle.edt_d2(oracle.seed_init(dn, en)))
+    codes = [oracle.march_level(field, en, i)[1].ravel() for i in range(L)]
+    irr = torch.empty((3, H, W), device="cuda:0")
+    before = (1, 1, 4) if march[2] == 1 else (1, 1, 1)
+    with rc.RadianceCascadeStage(W, H, levels=L) as st:
+        for order in range(6 if march[0] == 1 else 1):
+            st.set_march(*before)
+            for i in range(1, L):
+                st.set_march_order(i, 0)
+            st.run_device(d, e_lit, irr)
+            st.set_march(*march)
+            for i in range(1, L):
+                legal = not (order == 1 and 4 * 4 ** i < 16 or order == 4 and 4 * 4 ** i < 32)
+                st.set_march_order(i, order if legal else 0)
+            st.run_device(d, e, irr)
+            assert np.array_equal(irr.cpu().numpy().view(np.uint32), want.view(np.uint32)), order
+            for i in range(1, L):
+                n = rc.level_rays(W, H, i)
+                h = torch.empty(n, dtype=torch.int32, device="cuda:0")
+                ix = torch.empty(n, dtype=torch.int64, device="cuda:0")
+                st.debug_march(i, h, ix)
+                assert np.array_equal(h.cpu().numpy(), codes[i]), (order, i)
+                assert ix.min().item() >= 0 and torch.unique(ix).numel() == n, (order, i)
+                if st.march_order()[i] == 0:
+                    assert torch.equal(ix, torch.arange(n, device="cuda:0")), (order, i)
