@@ -704,7 +704,10 @@ def main():
                    "path": "plain", "launch": "direct (one stream)", "width": W, "height": H, "levels": L,
                    "storage": args.storage,
                    "rays_per_frame": int(sum(rays)),
-                   "tiling": {str(k): f"{v[0][0]}x{v[0][1]}x{v[0][2]} r{v[1]}" for k, v in tiling.items()},
+                   # the levels that run on a tile: those marched in place, and a top level the split march
+                   # does not merge (a level merged from stored codes has none)
+                   "tiling": {str(k): f"{v[0][0]}x{v[0][1]}x{v[0][2]} r{v[1]}" for k, v in tiling.items()
+                              if split == 0 or (k == L - 1 and not top_in_march)},
                    "march": {"split": split, "speculation": spec, "rays_per_lane": rpl, "top_level_merged": top_in_march,
                              "order": {str(k): v for k, v in stage.march_order().items()}},
                    "sdf": stage.sdf_mode(), "jfa_fuse": stage.jfa_fuse(), "jfa_rows": stage.jfa_rows()},

@@ -175,14 +175,21 @@ const char *rc_noalloc_last_error(void);
 void rc_destroy(rc_ctx *ctx);
 
 /* ---- level-kernel tiling (autotuner) ----------------------------------------
- * A level-i kernel (i >= 1) runs workgroups of TX x TY probes x KD directions
- * (TX*TY*KD = 256 lanes) with R rays per lane (probe rows TY apart).
+ * A level-i kernel (i >= 1) that marches its own rays (rc_set_march split = 0,
+ * and level 1 of the learned frame), or that merges a top level from stored
+ * codes, runs workgroups of TX x TY probes x KD directions (TX*TY*KD = 256
+ * lanes) with R rays per lane (probe rows TY apart).  After a split march a
+ * level with an upper one is merged without a tile, and the march itself merges
+ * the top level where it can (split = 1, one ray per lane, lane order not 5):
+ * there a level's tiling is kept, and has no effect until a mode uses it.
  * shape: 0 = 8x8x4, 1 = 4x4x16, 2 = 2x2x64, 3 = 1x1x256, 4 = 8x4x8 (TX x TY x KD;
  * KD <= N_i required);
  * rays_per_lane: 1, 2 or 4.  Every tiling computes identical results.
- * rc_autotune times every legal (shape, rays_per_lane) of every level on the
- * given device G-buffer (iters launches each, HIP events) and keeps the
- * fastest; rc_get_level_tiling reports the current choice. */
+ * rc_autotune picks the march mode and orders, times every legal (shape,
+ * rays_per_lane) of the levels that the picked mode runs on a tile (and of the
+ * top level after a split march) on the given device G-buffer (iters launches
+ * each, HIP events) and keeps the fastest; rc_get_level_tiling reports the
+ * current choice. */
 #define RC_NUM_TILE_SHAPES 5
 rc_status rc_set_level_tiling(rc_ctx *ctx, uint32_t level, uint32_t shape, uint32_t rays_per_lane);
 rc_status rc_get_level_tiling(const rc_ctx *ctx, uint32_t level, uint32_t *shape, uint32_t *rays_per_lane);
@@ -215,8 +222,9 @@ uint32_t rc_get_jfa_rows(const rc_ctx *ctx);
  * the same march by a persistent grid of resident waves, each walking an
  * interleaved share of 64-ray packets and handing a new ray to a lane as soon
  * as its ray ends (rays_per_lane must be 1); split = 0: each level kernel
- * marches and merges its own rays.  speculation (1, 2, 4) is the split
- * march's look-ahead depth; rays_per_lane (1, 2, 4, 8) how many rays a lane
+ * marches and merges its own rays.  speculation (2, 4) is the split march's
+ * look-ahead depth, 1 leaves it to the march (none at first, then where a
+ * wave's rays repeat their step); rays_per_lane (1, 2, 4, 8) how many rays a lane
  * of the split = 1 march takes one after another.  The result is identical;
  * rc_autotune also picks these (a one-level frame has nothing to march). */
 rc_status rc_set_march(rc_ctx *ctx, uint32_t split, uint32_t speculation, uint32_t rays_per_lane);
@@ -328,8 +336,8 @@ void rc_sha256(const void *data, uint64_t n, uint8_t *out32);
  * kernels (marched on a distance field exact up to 10 px).  Output 48
  * predicts log of the squared error.  Tiles of 8x8 level-2 probes whose mean
  * predicted error exceeds `threshold` take the plain cascades' level 1
- * (fallback: one full plain frame plus a patch, decided on the host after the
- * frame).  Needs levels >= 3. */
+ * (fallback: the plain levels of the probes those tiles need, marched, merged
+ * and patched in on the device within the frame).  Needs levels >= 3. */
 #define RC_MLP_INPUTS 64     /* per direction k: log(1 + c_k) rgb, cone transmittance T_k */
 #define RC_MLP_OUTPUTS 64
 #define RC_MLP_PARAMS 16640  /* for l = 0..3: W_l [K_l][64] (K = 64) then b_l [64] */

@@ -169,3 +169,32 @@ def test_every_form_and_order_marches_every_ray(rc, oracle, march, W, H, L):
                 assert ix.min().item() >= 0 and torch.unique(ix).numel() == n, (order, i)
                 if st.march_order()[i] == 0:
                     assert torch.equal(ix, torch.arange(n, device="cuda:0")), (order, i)
+
+
+@pytest.mark.parametrize("march,order", [((2, 1, 1), 0), ((1, 1, 2), 0), ((1, 1, 1), 5)])
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+def test_every_tiling_of_an_unmerged_top_level(rc, march, order, storage):
+    """The level kernel that reads stored codes runs only for a top level the
+    march does not merge: each of its tiles and rays per lane gives the frame
+    of the in-place march, after a frame in which every ray hits."""
+    W, H, L = 331, 190, 4
+    d, e = _boxes(rc, W, H, 6)
+    e_lit = torch.ones((3, H, W), device="cuda:0")
+    irr = torch.empty((3, H, W), device="cuda:0")
+    with rc.RadianceCascadeStage(W, H, levels=L, storage=storage) as st:
+        st.set_march(0, 1, 1)
+        st.run_device(d, e, irr)
+        want = irr.clone()
+        top = torch.empty(st.level_shape(L - 1), device="cuda:0")
+        st.debug_level(L - 1, top)
+        st.set_march_order(L - 1, order)
+        for shape in rc._abi.TILE_SHAPES:
+            for rpt in (1, 2, 4):
+                st.set_march(0, 1, 1)
+                st.run_device(d, e_lit, irr)
+                st.set_march(*march)
+                st.set_tiling(L - 1, shape, rpt)
+                st.run_device(d, e, irr)
+                got = torch.empty_like(top)
+                st.debug_level(L - 1, got)
+                assert torch.equal(got, top) and torch.equal(irr, want), (shape, rpt)
