@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "rc_internal.hpp"
+#include "rc_shuffle.hpp"
 
 namespace rc {
 
@@ -499,38 +500,17 @@ __global__ __launch_bounds__(kBlock) void k_mlp_refresh(MlpDev m)
 }
 
 // ---- the row order of an epoch ---------------------------------------------------
-// The Fisher-Yates shuffle of 0 .. n-1 that swaps position i with j_i = r_i
-// mod (i + 1) for i = n-1 .. 1, r the SplitMix64 stream after `state`, in
-// parallel and with the sequential loop's result.  At step i position i gets
-// its final value, the one position j_i holds, and the value of position i
-// moves to j_i.  So the value position p holds at step i was put there by the
-// latest earlier step that drew p, which is the smallest i' > i with j_i' =
-// p, or is p itself if there is none; and step i' moved the value position i'
-// held then, found the same way.  With the steps that drew p listed in
-// ascending order (the first kernel links them with one exchange each, the
-// second sorts each list: ln(n / p) steps on average), step i's predecessor is
-// the next in its own list, and the third kernel follows the predecessors to
-// a position nothing was moved into, a few hops.
+// The shuffle of rc_shuffle.hpp, a lane an element in each of its four steps.
 // The sequential loop on the host is a chain of cache misses: about 1.3 ms for
 // 524,288 rows (and 0.3 s for 16 M) with the upload; these four kernels take
 // 64 us.
-constexpr int kShuffleList = 24;  // steps of a list sorted in LDS; a longer one is sorted in place
-
-__device__ inline uint64_t splitmix64_at(uint64_t state, uint64_t k)
-{
-    uint64_t z = state + (k + 1) * 0x9E3779B97F4A7C15ull;
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    return z ^ (z >> 31);
-}
-
 __global__ __launch_bounds__(kBlock) void k_shuffle_clear(int *__restrict__ head, int n)
 {
     const int p = (int)(blockIdx.x * kBlock + threadIdx.x);
     if (p < n) head[p] = -1;
 }
 
-// Step i (1 .. n-1) takes draw n-1-i: order[i] = j_i, linked into list j_i.
+// order[i] = j_i, step i linked into list j_i.
 __global__ __launch_bounds__(kBlock) void k_shuffle_draw(uint64_t state, int n, int *__restrict__ order,
                                                          int *__restrict__ head, int *__restrict__ next)
 {
@@ -540,7 +520,7 @@ __global__ __launch_bounds__(kBlock) void k_shuffle_draw(uint64_t state, int n, 
         order[0] = 0;
         return;
     }
-    const int j = (int)(splitmix64_at(state, (uint64_t)(n - 1 - i)) % (uint64_t)(i + 1));
+    const int j = shuffle_target(state, n, i);
     order[i] = j;
     next[i] = atomicExch(&head[j], i);
 }
@@ -549,48 +529,15 @@ __global__ __launch_bounds__(kBlock) void k_shuffle_draw(uint64_t state, int n, 
 __global__ __launch_bounds__(kBlock) void k_shuffle_sort(int n, int *__restrict__ head, int *__restrict__ next)
 {
     __shared__ int buf[kShuffleList][kBlock];
-    const int p = (int)(blockIdx.x * kBlock + threadIdx.x), t = (int)threadIdx.x;
-    if (p >= n) return;
-    int len = 0, i = head[p];
-    for (; i >= 0 && len < kShuffleList; ++len) {
-        const int after = next[i];
-        int k = len;
-        for (; k > 0 && buf[k - 1][t] > i; --k) buf[k][t] = buf[k - 1][t];
-        buf[k][t] = i;
-        i = after;
-    }
-    if (len < 2 && i < 0) return;
-    head[p] = buf[0][t];
-    for (int k = 0; k < len; ++k) next[buf[k][t]] = k + 1 < len ? buf[k + 1][t] : -1;
-    while (i >= 0) {  // the rest, each put in its place in the list
-        const int after = next[i];
-        int before = -1, at = head[p];
-        while (at >= 0 && at < i) {
-            before = at;
-            at = next[at];
-        }
-        next[i] = at;
-        if (before < 0) head[p] = i;
-        else next[before] = i;
-        i = after;
-    }
+    const int p = (int)(blockIdx.x * kBlock + threadIdx.x);
+    if (p < n) shuffle_sort_list<kShuffleList>(p, head, next, &buf[0][threadIdx.x], kBlock);
 }
 
 __global__ __launch_bounds__(kBlock) void k_shuffle_resolve(int n, int *__restrict__ order,
                                                             const int *__restrict__ head, const int *__restrict__ next)
 {
     const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
-    if (i >= n) return;
-    // the step whose swap put the value there (position 0 has no step of its own)
-    int step = i == 0 ? head[0] : next[i];
-    if (step < 0) return;  // order[i] = j_i already
-    for (;;) {
-        const int first = head[step];
-        const int f = first != step ? first : next[step];  // a step may have drawn its own position
-        if (f < 0) break;
-        step = f;
-    }
-    order[i] = step;
+    if (i < n) shuffle_resolve(i, order, head, next);
 }
 
 hipError_t launch_shuffle(uint64_t state, size_t n, int *order, int *head, int *next, hipStream_t s)
