@@ -42,6 +42,7 @@ struct rc_ctx {
     int *dbg_codes = nullptr;
     size_t dbg_code_off[RC_MAX_LEVELS] = {};
     int code_src[RC_MAX_LEVELS] = {};
+    int graph_code_src[RC_MAX_LEVELS] = {};  // of the captured frame
     float2 *dirs = nullptr;
     size_t dir_off[RC_MAX_LEVELS] = {};
     int tile[RC_MAX_LEVELS] = {};
@@ -816,8 +817,12 @@ static rc_status run_frame_graph(rc_ctx *c, const float *depth, const float *emi
         c->g_key[0] = depth;
         c->g_key[1] = emissive;
         c->g_key[2] = irr;
+        std::copy(c->code_src, c->code_src + RC_MAX_LEVELS, c->graph_code_src);
     }
     HIP_TRY(c, hipGraphLaunch(c->gexec, s));
+    // the readbacks follow the replayed frame, whatever ran since its capture
+    std::copy(c->graph_code_src, c->graph_code_src + RC_MAX_LEVELS, c->code_src);
+    c->last_learned = c->surr_mode != 0;
     c->stats.runs += 1;
     c->ran = true;
     return RC_OK;

@@ -198,3 +198,34 @@ def test_every_tiling_of_an_unmerged_top_level(rc, march, order, storage):
                 got = torch.empty_like(top)
                 st.debug_level(L - 1, got)
                 assert torch.equal(got, top) and torch.equal(irr, want), (shape, rpt)
+
+
+def test_readbacks_follow_a_replayed_frame(rc):
+    """Training rows between two replays of a learned frame with a fallback:
+    the fallback's march has overwritten the rows' codes, so the readback
+    refuses them, as after a frame that is launched directly; and after a
+    replayed plain frame it returns that frame's levels."""
+    W, H, L = 240, 160, 4
+    d, e = _boxes(rc, W, H, 5)
+    d2, e2 = _boxes(rc, W, H, 6)
+    irr = torch.empty((3, H, W), device="cuda:0")
+    qy, qx = rc.probe_grid(W, H, 2)[::-1]
+    rows = torch.empty((qx * qy, 64), device="cuda:0"), torch.empty((qx * qy, 48), device="cuda:0")
+    codes = torch.empty(rc.level_rays(W, H, 2), dtype=torch.int32, device="cuda:0")
+    with rc.RadianceCascadeStage(W, H, levels=L, graph=True) as st, rc.RadianceCascadeStage(W, H, levels=L) as plain:
+        a2, want = torch.empty(st.level_shape(2), device="cuda:0"), torch.empty(st.level_shape(2), device="cuda:0")
+        plain.run_device(d, e, irr)
+        plain.debug_level(2, want)
+        st.load_weights()
+        st.set_surrogate(True, threshold=-1e30)
+        st.run_device(d, e, irr)
+        st.surrogate_samples(d2, e2, *rows)
+        st.run_device(d, e, irr)
+        with pytest.raises(rc.RcError):
+            st.debug_march(2, codes)
+        st.set_surrogate(False)
+        for _ in range(2):
+            st.run_device(d, e, irr)
+            st.debug_march(2, codes)
+            st.debug_level(2, a2)
+            assert torch.equal(a2, want)
