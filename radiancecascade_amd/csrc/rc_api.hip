@@ -359,7 +359,12 @@ static MarchAllArgs march_all_args(const rc_ctx *c, bool gated = false)
     }
     for (int j = 0; j < m.nlev; ++j) {
         march_level_blocks(m.lev[j], spec, rays, slots);
-        if (gated) m.lev[j].blocks = std::min(m.lev[j].blocks, std::max(1, kGatedWaves / m.nlev));
+        if (gated) {
+            MarchLevel &l = m.lev[j];
+            l.blocks = std::min(l.blocks, std::max(1, kGatedWaves / m.nlev));
+            l.stride = l.blocks;
+            l.packets = ((int)((l.slots + 63) >> 6) + l.blocks - 1) / l.blocks;
+        }
     }
     m.codes_base = c->codes;
     m.dirs_base = c->dirs;

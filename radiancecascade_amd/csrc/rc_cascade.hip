@@ -687,14 +687,18 @@ __device__ __forceinline__ bool ray_place(const RayOrder &o, const MarchLevel &L
     return px < o.PX && py < o.PY;
 }
 // The packets of wave `wave`: first, first + step, ... below end.  One ray a
-// lane at a time: a grid's width of waves apart; M: the M next to each other.
+// lane at a time: L.packets of them, L.stride apart, so that L.stride waves
+// share L.stride * L.packets; M: the M next to each other.
 struct Packets {
     int first, step, end;
 };
 __device__ __forceinline__ Packets wave_packets(const MarchLevel &L, int wave, int m)
 {
     const int all = uniform((int)((L.slots + 63) >> 6));
-    if (m == 1) return Packets{wave, uniform(L.blocks), all};
+    if (m == 1) {
+        const int stride = uniform(L.stride), first = wave + wave / stride * stride * (L.packets - 1);
+        return Packets{first, stride, uniform(min(all, first + stride * L.packets))};
+    }
     return Packets{wave * m, 1, min(wave * m + m, all)};
 }
 
@@ -780,10 +784,10 @@ __device__ __forceinline__ bool march_round(const SdfField &f, float cx, float c
 // two things bounded a launch of one packet per wave: handing out 163,200
 // one-wave workgroups takes 36 us alone (4.6 a ns), and a chain of 339
 // dependent samples of 0.17 us each takes as long as the whole launch, 58 us.
-// - A wave takes L.packets packets, a grid's width of waves apart (neighbouring
-//   packets hold rays of like length: 4 in a run gave one wave 4 long ones,
-//   66 us against 60), the next packet's directions read while the present one
-//   marches.
+// - A wave takes L.packets packets, L.stride apart, as a rule a grid's width of
+//   waves (neighbouring packets hold rays of like length: 4 in a run gave one
+//   wave 4 long ones, 66 us against 60), the next packet's directions read
+//   while the present one marches.
 // - A ray takes its first kMarchPlain samples one per step, in a branch-free
 //   divergent loop on the raw byte code (lanes leave as their rays end), and
 //   the rest kMarchTail at a time: 100 rounds instead of 339 samples for the
@@ -799,9 +803,7 @@ __device__ __forceinline__ bool march_round(const SdfField &f, float cx, float c
 //   samples one per step, probes again, and waits twice as long each time.
 //   That scene 373 us, lit boxes 122, 142 and 124 (121, 142 and 124 guessing
 //   always, 146 to 148 and 129 to 130 when the choice is made anew every round
-//   or few: it lies in the longest ray's chain).  What 8 packets a wave cost at
-//   3840x2160 stays: 2,960 us with a thousandth lit, 2,680 with 1, and boxes
-//   541 and 581.
+//   or few: it lies in the longest ray's chain).
 // Both kinds of scene with the field's zeros outside the image.
 constexpr int kMarchPlain = 16, kMarchTail = 4;
 constexpr int kTailProbe = 2, kTailShare = 16, kTailPlain = 32;
@@ -1344,6 +1346,7 @@ void march_level_map(MarchLevel &l, int map)
 void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64_t launch_slots)
 {
     l.packets = 1;
+    l.stride = 1;
     if (rays_per_lane == 1) {
         // few enough packets a wave that several times the 8,192 waves the chip
         // holds are left: with 1, 2, 4 and 8 a frame of 256x256 (4,096 packets) took
@@ -1352,9 +1355,22 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
         // 127.4 with 2 and 138.1 with 4, 3840x2160 (783,000) 553.9, 517.0, 506.8 and
         // 503.2, 16 views of 9.2 megapixels 900, 828, 792 and 772
         const int64_t n = launch_slots >> 6;
-        l.packets = n < 48 << 10 ? 1 : n < 192 << 10 ? 2 : n < 512 << 10 ? 4 : 8;
+        l.packets = n < 48 << 10 ? 1 : n < 192 << 10 ? 2 : n < 512 << 10 || l.map == 0 ? 4 : 8;
+        const int mine = (int)(((int64_t)l.slots + 63) >> 6);
+        l.stride = std::max(1, (mine + l.packets - 1) / l.packets);
+        // A launch of 8 in canonical order marches 8 parts of the image at a
+        // time, and a field of 8 MB does not stay in an L2 of 4 MB: there 512
+        // waves keep to 2,048 consecutive packets.  3840x2160 with a ten
+        // thousandth and a thousandth of the pixels lit 1,737 and 2,960 us with
+        // 8, 1,595 and 2,722 so (1,497 and 2,594 with one, before the tail
+        // guessed), four scenes of lit boxes 2,099 us together with 8, 2,067 so;
+        // 7680x4320 9,051 and 8,939.
+        if (n >= 512 << 10 && l.map == 0) l.stride = std::min(l.stride, 512);
+        const int group = l.stride * l.packets;
+        l.blocks = (mine + group - 1) / group * l.stride;
+        return;
     }
-    const int64_t per = (int64_t)kMarchBlock * rays_per_lane * l.packets;
+    const int64_t per = (int64_t)kMarchBlock * rays_per_lane;
     l.blocks = (int)(((int64_t)l.slots + per - 1) / per);
 }
 

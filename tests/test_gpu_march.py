@@ -133,13 +133,18 @@ def test_an_unused_fallback_costs_its_launches(rc):
     assert us[1e30] <= 1.4 * us[float("inf")], us
 
 
-@pytest.mark.parametrize("march", [(1, 1, 1), (1, 2, 1), (1, 4, 1), (1, 1, 2), (1, 2, 4), (1, 1, 8), (2, 1, 1)])
-@pytest.mark.parametrize("W,H,L", [(413, 211, 6), (97, 61, 4), (1030, 17, 3), (1366, 768, 6)])
-def test_every_form_and_order_marches_every_ray(rc, oracle, march, W, H, L):
+_FORMS = [(1, 1, 1), (1, 2, 1), (1, 4, 1), (1, 1, 2), (1, 2, 4), (1, 1, 8), (2, 1, 1)]
+
+
+@pytest.mark.parametrize("W,H,L,march", [(W, H, L, m) for W, H, L in ((413, 211, 6), (97, 61, 4), (1030, 17, 3),
+                                                                      (1366, 768, 6)) for m in _FORMS] +
+                         [(3801, 1900, 6, (1, 1, 1)), (3801, 1900, 6, (1, 2, 1))])
+def test_every_form_and_order_marches_every_ray(rc, oracle, W, H, L, march):
     """Each form of the split march in each order of its lanes, after another
     form left the codes and levels of a frame in which every ray hits: codes
     and irradiance are the oracle's, and the march's own packets place every
-    ray in one slot.  The larger size takes two packets a wave."""
+    ray in one slot.  The two larger sizes take several packets a wave, the
+    largest 4 that are 512 apart in canonical order and 8 in the others."""
     e_lit = torch.ones((3, H, W), device="cuda:0")
     d, e = _boxes(rc, W, H, 4)
     dn, en = d.cpu().numpy(), e.cpu().numpy()
