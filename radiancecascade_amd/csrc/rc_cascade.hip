@@ -687,8 +687,8 @@ __device__ __forceinline__ bool ray_place(const RayOrder &o, const MarchLevel &L
     return px < o.PX && py < o.PY;
 }
 // The packets of wave `wave`: first, first + step, ... below end.  One ray a
-// lane at a time: L.packets of them, L.stride apart, so that L.stride waves
-// share L.stride * L.packets; M: the M next to each other.
+// lane at a time: L.packets of them, L.stride apart, so that a group of L.stride
+// waves shares L.stride * L.packets; M: the M next to each other.
 struct Packets {
     int first, step, end;
 };
@@ -696,7 +696,8 @@ __device__ __forceinline__ Packets wave_packets(const MarchLevel &L, int wave, i
 {
     const int all = uniform((int)((L.slots + 63) >> 6));
     if (m == 1) {
-        const int stride = uniform(L.stride), first = wave + wave / stride * stride * (L.packets - 1);
+        const int before = wave >> L.group_log << L.group_log;  // waves in the groups before this one's
+        const int stride = uniform(L.stride), first = wave + before * (L.packets - 1);
         return Packets{first, stride, uniform(min(all, first + stride * L.packets))};
     }
     return Packets{wave * m, 1, min(wave * m + m, all)};
@@ -801,9 +802,10 @@ __device__ __forceinline__ bool march_round(const SdfField &f, float cx, float c
 //   kTailProbe rounds, and guesses on to the end of its rays if 1 in
 //   kTailShare of them had all four steps alike; otherwise it takes kTailPlain
 //   samples one per step, probes again, and waits twice as long each time.
-//   That scene 373 us, lit boxes 122, 142 and 124 (121, 142 and 124 guessing
-//   always, 146 to 148 and 129 to 130 when the choice is made anew every round
-//   or few: it lies in the longest ray's chain).
+//   (A launch too small to fill the chip, L.probe false, guesses always.)
+//   That scene 368 us; 8 scenes of lit boxes 118.7 us on average, 117.8 guessing
+//   always, and 6 to 20 us more where the choice is made anew every round: it
+//   lies in the longest ray's chain.
 // Both kinds of scene with the field's zeros outside the image.
 constexpr int kMarchPlain = 16, kMarchTail = 4;
 constexpr int kTailProbe = 2, kTailShare = 16, kTailPlain = 32;
@@ -819,6 +821,7 @@ __device__ __forceinline__ void march_packets(const SdfField &field, const March
     f.skip = uniform(f.skip);
     const RayOrder o = ray_order(L, lane);
     const int spacing = uniform((int)L.spacing);
+    const bool probe = L.probe;
     const float t0 = __int_as_float(uniform(__float_as_int(L.t0))), t1 = __int_as_float(uniform(__float_as_int(L.t1)));
     const float2 *dirs = L.dirs;
     int *codes = L.codes;
@@ -849,27 +852,33 @@ __device__ __forceinline__ void march_packets(const SdfField &field, const March
                 t = t + step_of_code(c);
                 alive = c != 0 && t < t1;
             }
-            int plain = kTailPlain;
-            while (const unsigned long long on = __ballot(alive)) {
-                int run = 0;
+            if (alive) {
+                int plain = kTailPlain;
                 bool all;
+                do {
+                    if (probe) {
+                        const int on = __popcll(__builtin_amdgcn_ballot_w64(true));
+                        bool run = false;
+#pragma unroll
+                        for (int round = 0; round < kTailProbe; ++round) {
+                            if (!alive) break;
+                            alive = march_round<kMarchTail>(f, cx, cy, dir, t1, t, guess, all);
+                            run = run || all;
+                        }
+                        if (__popcll(__builtin_amdgcn_ballot_w64(run)) * kTailShare < on) {
 #pragma unroll 1
-                for (int round = 0; alive && round < kTailProbe; ++round) {
-                    alive = march_round<kMarchTail>(f, cx, cy, dir, t1, t, guess, all);
-                    run = all ? 1 : run;
-                }
-                if (__popcll(__ballot(run != 0)) * kTailShare >= __popcll(on)) {
+                            for (int step = 0; alive && step < plain; ++step) {
+                                const uint32_t c = sdf_code(f, floor_i32(fmaf(t, dir.x, cx)), floor_i32(fmaf(t, dir.y, cy)));
+                                guess = step_of_code(c);
+                                t = t + guess;
+                                alive = c != 0 && t < t1;
+                            }
+                            plain *= 2;  // a ray takes fewer than 2^16 samples (t1 < 2^16, steps of 1 at least)
+                            continue;
+                        }
+                    }
                     while (alive) alive = march_round<kMarchTail>(f, cx, cy, dir, t1, t, guess, all);
-                    break;
-                }
-#pragma unroll 1
-                for (int step = 0; alive && step < plain; ++step) {
-                    const uint32_t c = sdf_code(f, floor_i32(fmaf(t, dir.x, cx)), floor_i32(fmaf(t, dir.y, cy)));
-                    guess = step_of_code(c);
-                    t = t + guess;
-                    alive = c != 0 && t < t1;
-                }
-                plain *= 2;  // a ray takes fewer than 2^16 samples (t1 < 2^16, steps of 1 at least)
+                } while (alive);
             }
         } else {
             bool all;
@@ -1347,6 +1356,8 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
 {
     l.packets = 1;
     l.stride = 1;
+    l.group_log = 31;
+    l.probe = false;
     if (rays_per_lane == 1) {
         // few enough packets a wave that several times the 8,192 waves the chip
         // holds are left: with 1, 2, 4 and 8 a frame of 256x256 (4,096 packets) took
@@ -1355,6 +1366,11 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
         // 127.4 with 2 and 138.1 with 4, 3840x2160 (783,000) 553.9, 517.0, 506.8 and
         // 503.2, 16 views of 9.2 megapixels 900, 828, 792 and 772
         const int64_t n = launch_slots >> 6;
+        // below this the chip is not full, loads are free and the longest ray is all:
+        // 8 scenes of lit boxes of 256x256 (4,096 packets) 32.7 us guessing always, 33.3
+        // probing; 700x300 (16,400) 49.9 and 49.8, with a thousandth of the pixels lit
+        // 58.0 and 52.9
+        l.probe = n >= 16 << 10;
         l.packets = n < 48 << 10 ? 1 : n < 192 << 10 ? 2 : n < 512 << 10 || l.map == 0 ? 4 : 8;
         const int mine = (int)(((int64_t)l.slots + 63) >> 6);
         l.stride = std::max(1, (mine + l.packets - 1) / l.packets);
@@ -1362,10 +1378,13 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
         // time, and a field of 8 MB does not stay in an L2 of 4 MB: there 512
         // waves keep to 2,048 consecutive packets.  3840x2160 with a ten
         // thousandth and a thousandth of the pixels lit 1,737 and 2,960 us with
-        // 8, 1,595 and 2,722 so (1,497 and 2,594 with one, before the tail
+        // 8, 1,593 and 2,717 so (1,497 and 2,594 with one, before the tail
         // guessed), four scenes of lit boxes 2,099 us together with 8, 2,067 so;
         // 7680x4320 9,051 and 8,939.
-        if (n >= 512 << 10 && l.map == 0) l.stride = std::min(l.stride, 512);
+        if (n >= 512 << 10 && l.map == 0 && l.stride > 512) {
+            l.stride = 512;
+            l.group_log = 9;
+        }
         const int group = l.stride * l.packets;
         l.blocks = (mine + group - 1) / group * l.stride;
         return;

@@ -228,7 +228,11 @@ struct MarchLevel {
     int map, tx_log, ty_log, kd_log, ntx;
     uint32_t rcp_ntx;        // ceil(2^32 / ntx), at most 2^32 - 1 (tile -> row, corrected)
     uint32_t slots;
-    int packets, stride;     // packets of 64 slots a wave marches one after another (one ray per lane), and how far apart
+    // one ray per lane: packets of 64 slots a wave marches one after another, how
+    // far apart, log2 of the waves whose packets interleave (31: all), and
+    // whether a wave probes before it guesses samples
+    int packets, stride, group_log;
+    bool probe;
     // The top level (no upper level) merged by the march itself: each lane
     // quad holds the 4 child directions of one texel, so the march writes
     // A_top = quad mean of (hit ? (E, 0) : (0, 1)) here, in `storage`
