@@ -1375,15 +1375,16 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
         const int mine = (int)(((int64_t)l.slots + 63) >> 6);
         l.stride = std::max(1, (mine + l.packets - 1) / l.packets);
         // A launch of 8 in canonical order marches 8 parts of the image at a
-        // time, and a field of 8 MB does not stay in an L2 of 4 MB: there 512
-        // waves keep to 2,048 consecutive packets.  3840x2160 with a ten
-        // thousandth and a thousandth of the pixels lit 1,737 and 2,960 us with
-        // 8, 1,593 and 2,717 so (1,497 and 2,594 with one, before the tail
-        // guessed), four scenes of lit boxes 2,099 us together with 8, 2,067 so;
-        // 7680x4320 9,051 and 8,939.
-        if (n >= 512 << 10 && l.map == 0 && l.stride > 512) {
-            l.stride = 512;
-            l.group_log = 9;
+        // time, and a field of 8 MB does not stay in an L2 of 4 MB: there 4,096
+        // waves keep to 16,384 consecutive packets.  3840x2160 with a ten
+        // thousandth and a thousandth of the pixels lit 1,736 and 2,954 us with
+        // 8, 1,585 and 2,731 so (1,492 and 2,586 with one, before the tail
+        // guessed), 16 scenes of lit boxes 524 us on average either way; with
+        // groups of 512 they took 534, with 1,024 to 8,192 and 8 packets 524 to
+        // 529.  7680x4320 2,261 us with 8, 2,231 so.
+        if (n >= 512 << 10 && l.map == 0 && l.stride > 4096) {
+            l.stride = 4096;
+            l.group_log = 12;
         }
         const int group = l.stride * l.packets;
         l.blocks = (mine + group - 1) / group * l.stride;

@@ -144,7 +144,7 @@ def test_every_form_and_order_marches_every_ray(rc, oracle, W, H, L, march):
     form left the codes and levels of a frame in which every ray hits: codes
     and irradiance are the oracle's, and the march's own packets place every
     ray in one slot.  The two larger sizes take several packets a wave, the
-    largest 4 that are 512 apart in canonical order and 8 in the others."""
+    largest 4 that are 4,096 apart in canonical order and 8 in the others."""
     e_lit = torch.ones((3, H, W), device="cuda:0")
     d, e = _boxes(rc, W, H, 4)
     dn, en = d.cpu().numpy(), e.cpu().numpy()
