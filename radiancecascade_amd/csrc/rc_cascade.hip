@@ -803,12 +803,12 @@ __device__ __forceinline__ bool march_round(const SdfField &f, float cx, float c
 //   kTailShare of them had all four steps alike; otherwise it takes kTailPlain
 //   samples one per step, probes again, and waits twice as long each time.
 //   (A launch too small to fill the chip, L.probe false, guesses always.)
-//   That scene 368 us; 8 scenes of lit boxes 118.7 us on average, 117.8 guessing
+//   That scene 373 us; 8 scenes of lit boxes 119.0 us on average, 118.3 guessing
 //   always, and 6 to 20 us more where the choice is made anew every round: it
 //   lies in the longest ray's chain.
 // Both kinds of scene with the field's zeros outside the image.
 constexpr int kMarchPlain = 16, kMarchTail = 4;
-constexpr int kTailProbe = 2, kTailShare = 16, kTailPlain = 32;
+constexpr int kTailProbe = 2, kTailShare = 16, kTailPlain = 24;
 
 template <int SPEC, bool GATED>
 __device__ __forceinline__ void march_packets(const SdfField &field, const MarchLevel &L, int lb,
