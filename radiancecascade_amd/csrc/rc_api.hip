@@ -357,15 +357,8 @@ static MarchAllArgs march_all_args(const rc_ctx *c, bool gated = false)
         l.dir_off = (int)c->dir_off[i];
         m.total_rays += (uint32_t)((int64_t)l.PX * l.PY * l.N);
     }
-    for (int j = 0; j < m.nlev; ++j) {
-        march_level_blocks(m.lev[j], spec, rays, slots);
-        if (gated) {
-            MarchLevel &l = m.lev[j];
-            l.blocks = std::min(l.blocks, std::max(1, kGatedWaves / m.nlev));
-            l.stride = l.blocks;
-            l.packets = ((int)((l.slots + 63) >> 6) + l.blocks - 1) / l.blocks;
-        }
-    }
+    for (int j = 0; j < m.nlev; ++j)
+        march_level_blocks(m.lev[j], spec, rays, slots, gated ? std::max(1, kGatedWaves / m.nlev) : 1 << 30);
     m.codes_base = c->codes;
     m.dirs_base = c->dirs;
     m.emis4 = c->emis4;

@@ -1352,7 +1352,7 @@ void march_level_map(MarchLevel &l, int map)
                        : (uint32_t)((int64_t)l.ntx * nty * (l.N >> l.kd_log) * 64);
 }
 
-void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64_t launch_slots)
+void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64_t launch_slots, int max_waves)
 {
     l.packets = 1;
     l.stride = 1;
@@ -1388,6 +1388,11 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
         }
         const int group = l.stride * l.packets;
         l.blocks = (mine + group - 1) / group * l.stride;
+        if (l.blocks > max_waves) {
+            l.blocks = l.stride = max_waves;
+            l.packets = (mine + max_waves - 1) / max_waves;
+            l.group_log = 31;
+        }
         return;
     }
     const int64_t per = (int64_t)kMarchBlock * rays_per_lane;

@@ -256,8 +256,9 @@ bool march_map_legal(int level, int map);
 inline int default_march_map(int level) { return num_dirs(level) >= 32 ? 4 : 0; }
 // fills map, the wave tile, ntx, rcp_ntx and slots of a level (PX, PY, N, log2n set)
 void march_level_map(MarchLevel &l, int map);
-// fills packets and blocks of a mapped level; launch_slots = the slots of every level (and view) of its launch
-void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64_t launch_slots);
+// fills packets, their stride and groups, and blocks of a mapped level; launch_slots = the slots of every level (and view) of its launch
+// (one ray per lane: at most max_waves waves, which then take more packets)
+void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64_t launch_slots, int max_waves = 1 << 30);
 struct MarchAllArgs {
     const uint8_t *sdf;
     int W, H, nlev;

@@ -86,10 +86,10 @@ def _boxes(rc, W, H, seed):
     return d, e
 
 
-@pytest.mark.parametrize("W,H,L", [(1366, 768, 6), (1921, 1079, 3)])
+@pytest.mark.parametrize("W,H,L", [(1366, 768, 6), (1921, 1079, 3), (3840, 2160, 7)])
 def test_fallback_march_of_several_packets_a_wave(rc, W, H, L):
-    """A fallback launch of more packets than its waves may be: flagged tiles
-    equal the plain level 1 bit for bit, the others the learned one, with
+    """A fallback launch of more packets than its waves may be (and of more than
+    512 K, where a plain frame's waves form groups): flagged tiles equal the plain level 1 bit for bit, the others the learned one, with
     another scene's codes left in the buffer."""
     irr = torch.empty((3, H, W), device="cuda:0")
     with rc.RadianceCascadeStage(W, H, levels=L) as plain, rc.RadianceCascadeStage(W, H, levels=L) as st:
