@@ -939,15 +939,18 @@ __global__ __launch_bounds__(kMarchBlock) void k_march_all(MarchAllArgs a)
 
 // The tile fallback's split march: nothing when no tile is flagged, and only
 // the probes the flagged tiles need.  A frame with no flagged tile pays for
-// handing the workgroups out, so there are few: two waves each, and at most
-// kGatedWaves waves a launch, which then take more packets.  Unused, with one
-// wave each and no limit, it took 60.2, 82.0, 110.3 and 283 us of frames of
-// 700x400, 1366x768, 1920x1080 and 3840x2160, 57.5, 77.0, 98.0 and 265 so
-// (56.4, 77.1, 99.9 and 288 when the fallback marched in place).  With about
-// 40 % of the tiles flagged 94.4, 136.3, 180.2 and 596 us, 94.1, 137.9, 182.0
-// and 592 so; with all of them 97.2, 145.4, 203 and 782, 97.0, 146.9, 213.5
-// and 785 (four waves and no limit: 97.4, 147.1, 213.5 and 807; 16,384 waves
-// of one: 98.9, 147.5, 211 and 806).
+// handing the workgroups out, so there are few: four waves each, and at most
+// kGatedWaves waves a launch, which then take more packets.  Means of 4 scenes,
+// in us, where the fallback marched level by level, with one wave a workgroup
+// and no limit, and so:
+//              no tile flagged       threshold 1         every tile
+//   700x400     56.2  60.3  56.1   136.9  94.3  94.5   150.6  98.6  98.0
+//   1366x768    79.0  83.1  76.9   201.1 127.3 128.3   255.7 148.2 148.9
+//   1920x1080  102.2 110.8  96.8   269.0 169.3 169.2   335.3 205.7 211.3
+//   3840x2160  283.9 278.0 261.8   742.7 511.4 514.7  1023.6 744.9 748.5
+// (two waves, 32,768 at most: 57.7, 78.6, 97.4 and 261 unused, 99.0, 149.1,
+// 209 and 742 with every tile; one wave, 32,768: 60.4, 82.9, 102.7 and 264
+// unused.)
 __global__ __launch_bounds__(kGatedBlock) void k_march_gated(MarchAllArgs a)
 {
     const MarchLevel &L = a.lev[blockIdx.y];

@@ -209,7 +209,7 @@ struct LevelArgs {
 };
 
 // the gated march: threads of a workgroup, and waves of a launch at most
-constexpr int kGatedBlock = 128, kGatedWaves = 32768;
+constexpr int kGatedBlock = 256, kGatedWaves = 65536;
 // k_march_all: every level >= 1 in one launch (level-major, top level first).
 struct MarchLevel {
     const float2 *dirs;
