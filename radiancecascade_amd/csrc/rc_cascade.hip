@@ -246,10 +246,11 @@ __global__ __launch_bounds__(kBlock) void k_level(LevelArgs a)
 // wave, without LDS or a barrier.  A quad of lanes holds the 4 children of the
 // 4 probes' next-lower direction: two exchanges leave lane q with probe q's sum
 // in the order (v0 + v1) + (v2 + v3), and every lane stores one texel.
-// Bound by latency and the hits' gathers: 24 us for the 4 merges of a lit
-// 1920x1080 frame (28 with the emission row by row), 45 in the staged form of
-// level_body (190 VALU per 128 rays, here 215 to 235 per 256 and 56 more in a
-// wave with a hit), 63 and 184 at 3840x2160 in half storage.
+// Bound by latency and the hits' gathers: 24 us for the 4 merges of a
+// 1920x1080 frame where a fifth of the pixels emit, 32 to 36 where more do (28
+// and 40 with the emission row by row), 45 in the staged form of level_body
+// (190 VALU per 128 rays, here 215 to 235 per 256 and 56 more in a wave with a
+// hit), 63 and 184 at 3840x2160 in half storage.
 __device__ inline float quad_exchange(float keep, float send, int ctrl_xor)
 {
     const int o = ctrl_xor == 1 ? __builtin_amdgcn_mov_dpp(__float_as_int(send), 0xB1, 0xF, 0xF, false)
@@ -1366,8 +1367,10 @@ void march_level_blocks(MarchLevel &l, int speculation, int rays_per_lane, int64
         // holds are left: with 1, 2, 4 and 8 a frame of 256x256 (4,096 packets) took
         // 32.2, 34.1, 38.4 and 48.2 us, 1283x717 (72,000) 89.6, 86.5, 87.9 and 93.8,
         // one scene of 1920x1080 (163,200) 133.1, 126.4, 125.7 and 130.0 and another
-        // 127.4 with 2 and 138.1 with 4, 3840x2160 (783,000) 553.9, 517.0, 506.8 and
-        // 503.2, 16 views of 9.2 megapixels 900, 828, 792 and 772
+        // 127.4 with 2 and 138.1 with 4, 6 scenes of 2200x1240 (216,000) 166.4, 160.1,
+        // 160.3 and 161.8, of 2560x1440 (351,000) 243.7, 228.6, 224.1 and 227.9,
+        // 3840x2160 (783,000) 553.9, 517.0, 506.8 and 503.2, 16 views of 9.2 megapixels
+        // 900, 828, 792 and 772
         const int64_t n = launch_slots >> 6;
         // below this the chip is not full, loads are free and the longest ray is all:
         // 8 scenes of lit boxes of 256x256 (4,096 packets) 32.7 us guessing always, 33.3
