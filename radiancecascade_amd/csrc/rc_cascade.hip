@@ -631,12 +631,14 @@ __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirs
 // are alike.  Canonical order is the wave tile of one probe x 64 directions,
 // or, for level 1's 16 directions (wrap), the canonical index itself: 4
 // consecutive probes, which may wrap to the next row.
-// A packet T is one wave-uniform tile (row, column, slice) and lane constants:
-// start points and addresses are a part of T's plus a lane's, and the level's
-// fields stay in scalar registers (read from the arguments per packet, one
-// after another, they took a launch without march and stores to 14.7 us at
-// 1920x1080).  Every march of the split launch and the readback of its order
-// place rays by this.
+// A packet T is one tile (row, column, slice) and lane constants: start points
+// and addresses are a part of T's, scalar where a wave takes one packet at a
+// time, plus a lane's, and the level's fields stay in scalar registers (read
+// from the arguments per packet, one after another, they took a launch without
+// march and stores to 14.7 us at 1920x1080).  Both forms of the split launch
+// and the readback of its order place rays by this (where a lane takes several
+// rays, T differs between lanes); the persistent form is canonical, by
+// decode_ray.
 struct RayOrder {
     int PX, PY, log2n, slots, tx_log, ty_log, ntx, rcp, kd_log, ns_log, smask;
     bool wrap;

@@ -171,12 +171,13 @@ __global__ __launch_bounds__(kInferLanes, 4) void k_mlp_infer(MlpDev m, const fl
 // chain of about a dozen barrier-separated LDS steps, so the aim is many
 // blocks in flight (64 KB of LDS: 2 workgroups, 8 waves per CU) and no global
 // round trip inside a block; after that the 66.5 KB of partial sums each
-// workgroup writes (34 MB for 16,384 samples).  The block size stays 32 samples
-// (and the partials one per block) because the gradient is defined as the sum
-// of the blocks' FP32 sums in block order.  Partials are written in the
-// accumulators' own order (dw_part_index), 1 KB per store, and put in master
-// order by the reduction.  16,384 samples: 85 us with one
-// wave per block (weights read from L2 per product, scalar LDS copies), 20 us so.
+// workgroup writes (34 MB for 16,384 samples).  The gradient is the sum of
+// the 32-sample blocks' FP32 sums in block order, one partial each: the same bits
+// whatever the grid.  Partials of several blocks would be fewer and another
+// rounding of the same sum.  They are written in the accumulators' own order
+// (part_to_master), 1 KB per store, and put in master order by the reduction.
+// 16,384 samples: 85 us with one wave per block (weights read from L2 per
+// product, scalar LDS copies), 20 us so.
 constexpr int kTrainRow = 64 + 1, kTrainTgt = kMlpRad + 1;
 
 // Where element i of a workgroup's partial belongs in the master vector: dW
